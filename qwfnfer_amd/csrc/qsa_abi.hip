@@ -787,7 +787,7 @@ int prefill_impl(const qwfn_qsa_shape *shape, const qwfn_kv_view *view, const Id
             e = launch_prefill_index(gp, *view, qb, nb, max_len, sb, nsb, sel_stride, w, st);
         }
         if (e != hipSuccess) return hip_fail(e, "prefill: indexer");
-        e = g.vdim ? launch_prefill_attention(gp, *view, qb, nb, sb, nsb, sel_stride, w.vmax, ob, st)
+        e = g.vdim ? launch_prefill_attention(gp, *view, qb, nb, n_q, sb, nsb, sel_stride, w.vmax, ob, st)
             : loop ? launch_dec_loop(gp, *view, qb, nb, max_len, sb, nsb, sel_stride, w.vmax, ob, st)
                    : launch_attention(gp, *view, qb, dummy_len, nb, max_len, sb, nsb, sel_stride, ob, w, st);
         if (e != hipSuccess) return hip_fail(e, "prefill: attention");

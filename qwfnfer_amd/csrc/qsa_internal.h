@@ -257,10 +257,13 @@ hipError_t launch_pf_approx_scores(const Geo &g, const qwfn_kv_view &v, const fl
 // The largest q8_0 V scale of each KV head over positions [0, n_pos) of
 // sequence g.pf_seq, as kVmaxWg partial maxima per head (vmax).
 hipError_t launch_prefill_vmax(const Geo &g, const qwfn_kv_view &v, int32_t n_pos, float *vmax, hipStream_t st);
-// Prefill attention on the matrix cores (block_tokens % 64 == 0): one wave
-// per (query, KV head) over its selection, no partials; vmax from
-// launch_prefill_vmax over every position the queries read.
-hipError_t launch_prefill_attention(const Geo &g, const qwfn_kv_view &v, const float *q, int32_t n_q,
+// Compute units of the current device (looked up once per device).
+int device_cus();
+// Prefill attention on the matrix cores (block_tokens % 64 == 0): one wave (a
+// call of few queries: several) per (query, KV head) over its selection, no
+// partials in memory; n_call: queries of the whole call this batch is part of;
+// vmax from launch_prefill_vmax over every position the queries read.
+hipError_t launch_prefill_attention(const Geo &g, const qwfn_kv_view &v, const float *q, int32_t n_q, int32_t n_call,
                                     const int32_t *sel, const int32_t *nsel, int32_t max_sel, const float *vmax,
                                     float *out, hipStream_t st);
 // Decode attention that makes its own selection from the scores of a

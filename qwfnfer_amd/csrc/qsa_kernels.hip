@@ -9,6 +9,7 @@
 #include <math.h>
 #include <stdint.h>
 
+#include <atomic>
 #include <type_traits>
 
 #include "qsa_append.h"
@@ -2627,18 +2628,25 @@ struct PfAttnLds {
 // Cells past the query's position have weight 0 and their V scale masked.
 // K and V tiles are addressed from a wave-uniform base plus a fixed per-lane
 // offset (no per-lane 64-bit address arithmetic per tile).
-template <int HD, int G>
+// SPLIT (few pairs): `split` waves of the workgroup share a pair, wave u of
+// them taking tiles u, u + split, ..., and add up their states through LDS at
+// the end (pf_split picks the count).
+template <int HD, int G, bool SPLIT>
 __global__ void __launch_bounds__((PfAttnCfg<HD, G>::WAVES * 64))
 k_pf_attn(Geo g, qwfn_kv_view v, const float *__restrict__ q, int32_t n_q, const int32_t *__restrict__ sel,
           const int32_t *__restrict__ nsel, int32_t max_sel, const float *__restrict__ vmax,
-          float *__restrict__ out) {
+          float *__restrict__ out, int32_t split) {
     using C = PfAttnCfg<HD, G>;
     constexpr int NJ = HD / 32, ND = HD / 16, NK4 = C::NK4, NS4 = C::NS4;
     static_assert(G <= 16, "one MFMA output column per query head");
     __shared__ PfAttnLds<HD, G> shw[C::WAVES];
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = threadIdx.x & 63;
-    const int pair = (int)blockIdx.x * C::WAVES + wv;
-    if (pair >= n_q * g.Hkv) return;                 // a whole wave; no workgroup barrier follows
+    const int nsp = SPLIT ? split : 1;               // waves a pair (divides WAVES)
+    const int sub = SPLIT ? wv % nsp : 0;            // this wave's place among them
+    int pair = SPLIT ? (int)blockIdx.x * (C::WAVES / nsp) + wv / nsp : (int)blockIdx.x * C::WAVES + wv;
+    const bool live = pair < n_q * g.Hkv;
+    if (!SPLIT && !live) return;                     // a whole wave; no workgroup barrier follows
+    if (SPLIT && !live) pair = n_q * g.Hkv - 1;      // (walks no tile and writes nothing)
     PfAttnLds<HD, G> &W = shw[wv];
     const int s = pair / g.Hkv, gh = pair - s * g.Hkv;
     const int L = g.pf_pos0 + s + 1;
@@ -2725,7 +2733,9 @@ k_pf_attn(Geo g, qwfn_kv_view v, const float *__restrict__ q, int32_t n_q, const
     // running max starts at a finite floor far below any score, so exp2 of
     // (score - max) never sees inf - inf
     float m = -1e30f, lsum = 0.0f;                   // lsum in units of 2^kup
-    const int n_tiles = n * tpb;
+    // this wave's tiles: tile sub + nsp t of the pair is its tile t
+    const int all_tiles = live ? n * tpb : 0;
+    const int n_tiles = SPLIT ? (max(all_tiles - sub, 0) + nsp - 1) / nsp : all_tiles;
     // lane l's 16 bytes of a V tile's 1 KB transfer: dim row l / 4, quarter
     // (l % 4) ^ (row / 4 % 4)
     const uint32_t v_lane = (uint32_t)((l >> 2) * 64 + (((l & 3) ^ ((l >> 4) & 3)) << 4));
@@ -2734,8 +2744,8 @@ k_pf_attn(Geo g, qwfn_kv_view v, const float *__restrict__ q, int32_t n_q, const
         // query -- looked up for 64 tiles at once, read back per tile by readlane
         int pg_l = 0, r0_l = 0, nv_l = 0;
         {
-            const int t = tc + l;
-            if (t < n_tiles) {
+            if (tc + l < n_tiles) {
+                const int t = SPLIT ? sub + nsp * (tc + l) : tc + l;
                 const int blk = selp[t / tpb];
                 const int64_t t0 = (int64_t)blk * g.bt + (t % tpb) * 64;
                 if (blk >= 0 && t0 < L) {
@@ -3001,6 +3011,44 @@ k_pf_attn(Geo g, qwfn_kv_view v, const float *__restrict__ q, int32_t n_q, const
 #pragma unroll
             for (int i = 0; i < 4; ++i) o[d][i] += dppf<kDppRowRor8>(0.0f, o[d][i]);
     }
+    if constexpr (SPLIT) {
+        // the pair's waves: (max, sum) of each head through the weight strips,
+        // then each wave's O, weighted to the common maximum, over its own tile
+        // buffer (every transfer into it has landed and been read), and the
+        // waves add up a share of the row each, in wave order
+        static_assert(G * HD * 4 <= C::BUF16 * 16, "a wave's O fits its tile buffer");
+        const int w0 = wv - sub;
+        if (hv && lg == 0) {
+            W.p[hn][0] = m;
+            W.p[hn][1] = lsum;
+        }
+        __syncthreads();
+        if (hv) {
+            float mx = m;
+            for (int u = 0; u < nsp; ++u) mx = fmaxf(mx, shw[w0 + u].p[hn][0]);
+            const float wt = __builtin_amdgcn_exp2f(m - mx);
+            float *ow = reinterpret_cast<float *>(&W.buf[0]) + hn * HD;
+#pragma unroll
+            for (int d = 0; d < ND; ++d)
+                *reinterpret_cast<f4v *>(ow + 16 * d + 4 * lg) = o[d] * wt;
+        }
+        __syncthreads();
+        if (!live) return;
+        for (int i = 64 * sub + l; i < G * HD / 4; i += 64 * nsp) {      // four dims of head h
+            const int h = 4 * i / HD;
+            float mx = -INFINITY;
+            for (int u = 0; u < nsp; ++u) mx = fmaxf(mx, shw[w0 + u].p[h][0]);
+            float ls = 0.0f;
+            f4v t = {0.0f, 0.0f, 0.0f, 0.0f};
+            for (int u = 0; u < nsp; ++u) {
+                ls = __builtin_fmaf(shw[w0 + u].p[h][1], __builtin_amdgcn_exp2f(shw[w0 + u].p[h][0] - mx), ls);
+                t += reinterpret_cast<const f4v *>(&shw[w0 + u].buf[0])[i];
+            }
+            const float inv = ls > 0.0f ? 1.0f / ls : 0.0f;
+            reinterpret_cast<f4v *>(out + ((int64_t)s * g.H + gh * G) * HD)[i] = t * inv;
+        }
+        return;
+    }
     if (hv) {
         const float inv = lsum > 0.0f ? 1.0f / lsum : 0.0f;
         float *orow = out + ((int64_t)s * g.H + gh * G + hn) * HD;
@@ -3011,22 +3059,65 @@ k_pf_attn(Geo g, qwfn_kv_view v, const float *__restrict__ q, int32_t n_q, const
     }
 }
 
+int device_cus() {
+    static std::atomic<int> cache[64];
+    int dev = -1;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+    int n = cache[dev].load(std::memory_order_relaxed);
+    if (n <= 0) {
+        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) return 256;
+        cache[dev].store(n, std::memory_order_relaxed);
+    }
+    return n;
+}
+
+// Waves that share a (query, KV head) pair of the prefill attention, a power of
+// two up to a workgroup's `waves`: the count with the shortest estimated run,
+// workgroup rounds over the device's CUs (one workgroup fills a CU's LDS) times
+// the tiles a wave walks, plus two tiles' time for a wave's start (and merge).
+// A chunk of thousands of queries fills the chip with one wave a pair (and its
+// tiles then need no merge); a short one leaves CUs idle behind 73 tiles in
+// series.  `pairs` is the whole call's, so the query batches of a call
+// agree on the count (the result does not depend on the batch).  Measured: 203
+// queries after 32,700 tokens 334 -> 133 us a call (four waves a pair; the
+// attention itself 283 -> 82 us); 8,192 queries keep one wave a pair (2.80 ms).
+static int pf_split(int64_t pairs, int waves, int tiles) {
+    const int cus = device_cus();
+    int best = 1;
+    int64_t best_cost = 0;
+    for (int s = 1; s <= waves && waves % s == 0; s *= 2) {
+        const int64_t wgs = (pairs * s + waves - 1) / waves;
+        const int64_t cost = ((wgs + cus - 1) / cus) * ((tiles + s - 1) / s + 2);
+        if (s == 1 || cost < best_cost) {
+            best = s;
+            best_cost = cost;
+        }
+    }
+    return best;
+}
+
 template <int HD, int G>
-static void launch_pf_attn_t(const Geo &g, const qwfn_kv_view &v, const float *q, int32_t n_q,
+static void launch_pf_attn_t(const Geo &g, const qwfn_kv_view &v, const float *q, int32_t n_q, int32_t n_call,
                              const int32_t *sel, const int32_t *nsel, int32_t max_sel, const float *vmax,
                              float *out, hipStream_t st) {
     constexpr int WAVES = PfAttnCfg<HD, G>::WAVES;
     const int pairs = n_q * g.Hkv;
-    hipLaunchKernelGGL((k_pf_attn<HD, G>), dim3((unsigned)((pairs + WAVES - 1) / WAVES)), dim3(WAVES * 64), 0, st, g,
-                       v, q, n_q, sel, nsel, max_sel, vmax, out);
+    const int split = pf_split((int64_t)n_call * g.Hkv, WAVES, max_sel * (g.bt / 64));
+    const dim3 grid((unsigned)((pairs * split + WAVES - 1) / WAVES));
+    if (split == 1)
+        hipLaunchKernelGGL((k_pf_attn<HD, G, false>), grid, dim3(WAVES * 64), 0, st, g, v, q, n_q, sel, nsel, max_sel,
+                           vmax, out, 1);
+    else
+        hipLaunchKernelGGL((k_pf_attn<HD, G, true>), grid, dim3(WAVES * 64), 0, st, g, v, q, n_q, sel, nsel, max_sel,
+                           vmax, out, split);
 }
 
-hipError_t launch_prefill_attention(const Geo &g, const qwfn_kv_view &v, const float *q, int32_t n_q,
+hipError_t launch_prefill_attention(const Geo &g, const qwfn_kv_view &v, const float *q, int32_t n_q, int32_t n_call,
                                     const int32_t *sel, const int32_t *nsel, int32_t max_sel, const float *vmax,
                                     float *out, hipStream_t st) {
 #define X(HD_, G_, TG_)                                                                          \
     if (g.hd == HD_ && g.G == G_) {                                                              \
-        launch_pf_attn_t<HD_, G_>(g, v, q, n_q, sel, nsel, max_sel, vmax, out, st);             \
+        launch_pf_attn_t<HD_, G_>(g, v, q, n_q, n_call, sel, nsel, max_sel, vmax, out, st);     \
         return hipGetLastError();                                                                \
     }
     QWFN_FOR_EACH_SHAPE(X)
