@@ -9,6 +9,7 @@
 #include <math.h>
 #include <stdint.h>
 
+#include <algorithm>
 #include <atomic>
 #include <type_traits>
 
@@ -2422,6 +2423,18 @@ k_pf_refine_big(Geo g, qwfn_kv_view v, const float *__restrict__ q, float *score
     emit_forced<NT>(g, r, topk, out);
 }
 
+// k_pf_approx's grid over n_elig blocks of n_rows score rows a query: `split`
+// workgroups a query tile for calls that fill the chip (the measured best of
+// many queries), more, down to one 64-block tile each, while the grid stays
+// within two workgroups a CU: a call of few queries otherwise walks its block
+// tiles in series on a few CUs (203 queries over 511 blocks: 16 workgroups of 4
+// tiles took 24.0 us, 64 of one tile 14.0).
+static dim3 pa_grid(int n_q, int n_elig, int n_rows, int split) {
+    const int qt = (n_q + kPaQ - 1) / kPaQ, tiles = (n_elig + kPaB - 1) / kPaB;
+    const int fill = 2 * device_cus() / (qt * n_rows);
+    return dim3((unsigned)qt, (unsigned)std::max(split, std::min(tiles, fill)), (unsigned)n_rows);
+}
+
 template <int HD, int G>
 static void launch_pf_approx(const Geo &g, dim3 grid, const qwfn_kv_view &v, const float *q, int32_t n_q,
                              int32_t n_blk, float *scores, int32_t nb_cap, float *pnorm, hipStream_t st) {
@@ -2443,16 +2456,16 @@ static void launch_pf_index_t(const Geo &g, const qwfn_kv_view &v, const float *
         // to kRbBlocks eligible blocks: the 1024-thread refinement
         if (g.Hkv == 1 && g.topk > 0 && n_blk > g.sink && n_blk - g.sink > kRefineBlocks &&
             n_blk - g.sink <= kRbBlocks) {
-            launch_pf_approx<HD, G>(g, dim3((unsigned)((n_q + kPaQ - 1) / kPaQ), (unsigned)kPaSplitBig, 1u), v, q, n_q,
-                                    n_blk, ws.scores, ws.nb_cap, ws.pnorm, st);
+            launch_pf_approx<HD, G>(g, pa_grid(n_q, n_blk - g.sink, 1, kPaSplitBig), v, q, n_q, n_blk, ws.scores,
+                                    ws.nb_cap, ws.pnorm, st);
             hipLaunchKernelGGL((k_pf_refine_big<HD, G>), dim3(1u, (unsigned)n_q), dim3(kRbThreads), 0, st, g, v, q,
                                ws.scores, ws.nb_cap, ws.pnorm, sel, nsel, max_sel);
             return;
         }
         // per-KV-head selections (or one KV head's row shared), up to kRefineBlocks eligible blocks
         if ((!g.shared || g.Hkv == 1) && g.topk > 0 && n_blk > g.sink && n_blk - g.sink <= kRefineBlocks) {
-            launch_pf_approx<HD, G>(g, dim3((unsigned)((n_q + kPaQ - 1) / kPaQ), (unsigned)kPaSplit, (unsigned)g.Hkv),
-                                    v, q, n_q, n_blk, ws.scores, ws.nb_cap, ws.pnorm, st);
+            launch_pf_approx<HD, G>(g, pa_grid(n_q, n_blk - g.sink, g.Hkv, kPaSplit), v, q, n_q, n_blk, ws.scores,
+                                    ws.nb_cap, ws.pnorm, st);
             hipLaunchKernelGGL((k_pf_refine<HD, G>), dim3((unsigned)g.Hkv, (unsigned)n_q), dim3(kIdxThreads), 0, st, g,
                                v, q, ws.scores, ws.nb_cap, ws.pnorm, sel, nsel, max_sel);
             return;
@@ -3080,7 +3093,7 @@ int device_cus() {
 // series.  `pairs` is the whole call's, so the query batches of a call
 // agree on the count (the result does not depend on the batch).  Measured: 203
 // queries after 32,700 tokens 334 -> 133 us a call (four waves a pair; the
-// attention itself 283 -> 82 us); 8,192 queries keep one wave a pair (2.80 ms).
+// attention itself 283 -> 88 us); 8,192 queries keep one wave a pair (2.80 ms).
 static int pf_split(int64_t pairs, int waves, int tiles) {
     const int cus = device_cus();
     int best = 1;
