@@ -768,11 +768,17 @@ int prefill_impl(const qwfn_qsa_shape *shape, const qwfn_kv_view *view, const Id
         e = launch_prefill_vmax(gp, *view, max_len, w.vmax, st);
         if (e != hipSuccess) return hip_fail(e, "prefill: V scales");
     }
-    for (int32_t i0 = 0; i0 < n_q; i0 += batch) {
+    // the leading queries that attend every block up to their position share
+    // tiles and need no selection (their batch size is not the workspace's)
+    const int32_t n_full = parts ? 0 : pf_full_queries(gp, pos0, n_q);
+    if (n_full > 0) {
+        gp.pf_pos0 = pos0;
+        e = launch_prefill_full(gp, *view, q, n_full, w.vmax, out, st);
+        if (e != hipSuccess) return hip_fail(e, "prefill: attention over every block");
+    }
+    for (int32_t i0 = sel_out ? 0 : n_full; i0 < n_q; i0 += batch) {
         const int32_t nb = std::min(batch, n_q - i0);
         gp.pf_pos0 = pos0 + i0;
-        const float *qb = q + (int64_t)i0 * g.H * g.hd;
-        float *ob = out + (int64_t)i0 * g.H * g.hd;
         int32_t *sb = sel_out ? sel_out + (int64_t)i0 * g.Hkv * sel_stride : w.sel;
         int32_t *nsb = n_sel_out ? n_sel_out + (int64_t)i0 * g.Hkv : w.nsel;
         // prefill mode ignores the seq_len value; the pointer only has to be
@@ -784,12 +790,20 @@ int prefill_impl(const qwfn_qsa_shape *shape, const qwfn_kv_view *view, const Id
             const float *qib = ix->q_idx + (int64_t)i0 * gi.H * gi.hd;
             e = launch_prefill_index(gi, ix->vi, qib, nb, max_len, sb, nsb, sel_stride, w, st);
         } else {
-            e = launch_prefill_index(gp, *view, qb, nb, max_len, sb, nsb, sel_stride, w, st);
+            e = launch_prefill_index(gp, *view, q + (int64_t)i0 * g.H * g.hd, nb, max_len, sb, nsb, sel_stride, w, st);
         }
         if (e != hipSuccess) return hip_fail(e, "prefill: indexer");
-        e = g.vdim ? launch_prefill_attention(gp, *view, qb, nb, n_q, sb, nsb, sel_stride, w.vmax, ob, st)
-            : loop ? launch_dec_loop(gp, *view, qb, nb, max_len, sb, nsb, sel_stride, w.vmax, ob, st)
-                   : launch_attention(gp, *view, qb, dummy_len, nb, max_len, sb, nsb, sel_stride, ob, w, st);
+        // the batch's queries past those (a selection asked for takes in all)
+        const int32_t skip = std::max(0, n_full - i0), na = nb - skip;
+        if (na <= 0) continue;
+        gp.pf_pos0 += skip;
+        const float *qb = q + (int64_t)(i0 + skip) * g.H * g.hd;
+        float *ob = out + (int64_t)(i0 + skip) * g.H * g.hd;
+        sb += (int64_t)skip * g.Hkv * sel_stride;
+        nsb += (int64_t)skip * g.Hkv;
+        e = g.vdim ? launch_prefill_attention(gp, *view, qb, na, n_q - n_full, sb, nsb, sel_stride, w.vmax, ob, st)
+            : loop ? launch_dec_loop(gp, *view, qb, na, max_len, sb, nsb, sel_stride, w.vmax, ob, st)
+                   : launch_attention(gp, *view, qb, dummy_len, na, max_len, sb, nsb, sel_stride, ob, w, st);
         if (e != hipSuccess) return hip_fail(e, "prefill: attention");
     }
     return ok();

@@ -266,6 +266,13 @@ int device_cus();
 hipError_t launch_prefill_attention(const Geo &g, const qwfn_kv_view &v, const float *q, int32_t n_q, int32_t n_call,
                                     const int32_t *sel, const int32_t *nsel, int32_t max_sel, const float *vmax,
                                     float *out, hipStream_t st);
+// Prefill attention of queries that attend every block up to their position,
+// a block of queries sharing each tile (qsa_prefill_full.hip).
+// pf_full_queries: how many leading queries of a call do (0 for a shape
+// without an instance); vmax from launch_prefill_vmax (unused for F16).
+int32_t pf_full_queries(const Geo &g, int32_t pos0, int32_t n_q);
+hipError_t launch_prefill_full(const Geo &g, const qwfn_kv_view &v, const float *q, int32_t n_q, const float *vmax,
+                               float *out, hipStream_t st);
 // Decode attention that makes its own selection from the scores of a
 // scores-only indexer launch, writing it to sel / nsel (the q8_0 matrix-core
 // kernel for its shapes, the general kernel for the other element types and

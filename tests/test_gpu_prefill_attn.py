@@ -1,8 +1,13 @@
 """The prefill attention's launch variants against the oracle (the cases,
 checks and tolerance of test_gpu_parity's _prefill_case)."""
+import numpy as np
 import pytest
+import torch
 
+from _ckpt import CKPT
+from _gpu import assert_close_attn, cfg_of, kv_rows, np_of
 from _refs import BASELINE, Cfg
+from qwfnfer_amd import qsa
 from test_gpu_parity import _prefill_case
 
 pytestmark = pytest.mark.gpu
@@ -19,3 +24,76 @@ pytestmark = pytest.mark.gpu
 ])
 def test_prefill_few_queries(cfg, pre, n_q):
     _prefill_case(cfg, pre, n_q, seed=700 + n_q)
+
+
+# Queries that attend every block (a prompt's first thousands, a dense layer),
+# taken a block of queries at a time: counts that leave a partial query block and
+# tile, chunks from the first token and from inside a tile, one that ends past the
+# last such query (the rest selects), both group counts a workgroup, each layout.
+@pytest.mark.parametrize("cfg, pre, n_q", [
+    (BASELINE, 0, 515), (BASELINE, 37, 1030), (BASELINE, 4000, 850), (BASELINE, 0, 1),
+    (Cfg(top_k_blocks=0), 5001, 520),
+    (Cfg(head_dim=64), 3, 600), (Cfg(head_dim=256), 64, 530), (Cfg(n_head=8), 10, 540), (Cfg(n_head=4), 10, 540),
+    (Cfg(n_head=24, head_dim=256), 100, 520),
+    (Cfg(kv_type=1), 5, 420), (Cfg(kv_type=2), 63, 400), (Cfg(kv_type=2, block_tokens=16, top_k_blocks=300), 1, 401),
+    (CKPT, 129, 390),
+])
+def test_prefill_every_block(cfg, pre, n_q):
+    _prefill_case(cfg, pre, n_q, seed=800 + n_q, dtype=np.float16 if n_q % 2 else np.float32)
+
+
+def _chunk(cfg, pre, n_q, seed, edit=None, sel=False, q_batch=None):
+    """Output of a chunk over seeded rows (a row of the chunk's V changed by `edit`)."""
+    c = cfg_of(cfg)
+    rng = np.random.default_rng(seed)
+    k, v = kv_rows(rng, pre + n_q, cfg)
+    q = torch.from_numpy(rng.standard_normal((n_q, cfg.n_head, cfg.head_dim), dtype=np.float32)).cuda()
+    if edit:
+        edit(v)
+    dev = qsa.KvCache.allocate(c, 1, (pre + n_q) // cfg.page_tokens + 1)
+    kd, vd = torch.from_numpy(k).cuda(), torch.from_numpy(v).cuda()
+    if pre:
+        qsa.append_q8_0(dev, kd[:pre], vd[:pre], torch.arange(pre, dtype=torch.int32, device="cuda"))
+        qsa.pool_rebuild(dev, 0, pre // cfg.block_tokens)
+    ws = qsa.Workspace.for_prefill(c, pre + n_q, q_batch or n_q)
+    s = n = None
+    if sel:
+        s = torch.empty((n_q, cfg.n_head_kv, c.max_selected(pre + n_q)), dtype=torch.int32, device="cuda")
+        n = torch.empty((n_q, cfg.n_head_kv), dtype=torch.int32, device="cuda")
+    out = qsa.sparse_attn_prefill(dev, q, 0, pre, ws, kd[pre:].contiguous(), vd[pre:].contiguous(), sel=s, n_sel=n)
+    torch.cuda.synchronize()
+    return np_of(out)
+
+
+def test_prefill_every_block_selection_and_batches_are_invisible():
+    """The same bytes whether the selection is asked for or not, and whatever
+    batch the workspace holds, over a chunk that ends past the last query that
+    attends every block."""
+    a = _chunk(BASELINE, 4000, 850, 90)
+    np.testing.assert_array_equal(a, _chunk(BASELINE, 4000, 850, 90, sel=True))
+    np.testing.assert_array_equal(a, _chunk(BASELINE, 4000, 850, 90, sel=True, q_batch=100))
+    np.testing.assert_array_equal(a, _chunk(BASELINE, 4000, 850, 90, q_batch=100))
+
+
+@pytest.mark.parametrize("kv_type", [0, 1, 2])
+@pytest.mark.parametrize("bad", [300, 575, 511])
+def test_prefill_every_block_non_finite_rows(kv_type, bad):
+    """A non-finite V row reaches the queries at and after its position (the dims
+    of its 32-value block, NaN or infinite) and no earlier one, wherever it lies in its
+    tile and query block."""
+    cfg = Cfg(kv_type=kv_type)
+    n_q = 576
+
+    def edit(v):
+        v[bad, 1, 40] = np.inf                       # block 1 of KV head 1
+
+    dims = slice(32, 64) if kv_type != 2 else slice(40, 41)   # a quantized block shares its scale
+
+    def zero(v):                                     # the reference run: the key stays, those values are 0
+        v[bad, 1, dims] = 0.0
+
+    got, ref = _chunk(cfg, 0, n_q, 91, edit), _chunk(cfg, 0, n_q, 91, zero)
+    G = cfg.n_head // cfg.n_head_kv
+    assert not np.isfinite(got[bad:, G:, dims]).any()
+    got[bad:, G:, dims], ref[bad:, G:, dims] = 0.0, 0.0
+    assert_close_attn(got, ref.astype(np.float64))
