@@ -221,7 +221,9 @@ int qwfn_qsa_pooled_bytes(const qwfn_qsa_shape *shape, int32_t n_seq,
 int qwfn_qsa_max_selected(const qwfn_qsa_shape *shape, int32_t max_seq_len,
                           int32_t *max_sel);
 /* Workspace for qwfn_indexer_topk / qwfn_sparse_decode_attn /
- * qwfn_sparse_attn_decode at n_seq sequences up to max_seq_len tokens.  The
+ * qwfn_sparse_attn_decode at n_seq sequences up to max_seq_len tokens, with
+ * room (for up to eight sequences) for 8 n_seq, at most 16, rows of
+ * qwfn_sparse_attn_decode_chain to go out together; a call needs less.  The
  * workspace carries completion counters that every call leaves at zero:
  * initialise a new workspace once with qwfn_qsa_workspace_init (a fill kernel,
  * not a memset, so it may also be captured).  Calls that overlap on one
@@ -361,9 +363,13 @@ int qwfn_sparse_attn_decode(const qwfn_qsa_shape *shape, const qwfn_kv_view *vie
  * [n_pos][n_seq][n_head][head_dim], sel_out [n_pos][n_seq][n_head_kv]
  * [qwfn_qsa_max_selected] and n_sel_out [n_pos][n_seq][n_head_kv] (optional).
  * max_seq_len bounds seq_len + n_pos - 1.  One small launch derives the
- * positions' lengths into the workspace, then each position makes
- * qwfn_sparse_attn_decode's launches; all on `stream`, so the chain captures
- * into one hipGraph.  n_pos = 1 is qwfn_sparse_attn_decode.                   */
+ * positions' lengths into the workspace.  The positions then go out together,
+ * as rows of one scoring, one attention and one merge launch and a pooling of
+ * the blocks they complete, as many at a time as the workspace holds, where the
+ * attention selects for itself (qwfn_sparse_attn_decode) and local_tokens >=
+ * n_pos; else each position makes qwfn_sparse_attn_decode's launches in turn.
+ * The results are the same.  All on `stream`, so the chain captures into one
+ * hipGraph.  n_pos = 1 is qwfn_sparse_attn_decode.                            */
 int qwfn_sparse_attn_decode_chain(const qwfn_qsa_shape *shape, const qwfn_kv_view *view,
                                   const float *q, const void *k_new, const void *v_new,
                                   int32_t src_dtype, const int32_t *seq_len, int32_t n_seq,

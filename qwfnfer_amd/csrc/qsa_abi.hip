@@ -121,7 +121,7 @@ int make_geo(const qwfn_qsa_shape *s, const qwfn_kv_view *v, Geo *g, bool view_r
     // element types run the general kernels over the K layout
     g->vdim = s->block_tokens % 64 == 0 && s->kv_type == QWFN_KV_Q8_0;
     g->scale_log2 = (float)(1.4426950408889634 / std::sqrt((double)s->head_dim));
-    g->pf = 0; g->pf_seq = 0; g->pf_pos0 = 0;
+    g->pf = 0; g->pf_seq = 0; g->pf_pos0 = 0; g->chain = 0;
     g->pooled_f16 = 0;
     if (v) {
         g->pps = v->pages_per_seq; g->n_phys = v->n_phys_pages; g->n_seq_view = v->n_seq;
@@ -138,6 +138,19 @@ int32_t max_selected(const qwfn_qsa_shape *s, int32_t max_seq_len) {
     const int32_t win = (s->local_tokens + bt - 2) / bt + 1;
     const int64_t cap = (int64_t)s->top_k_blocks + s->sink_blocks + win;
     return cap < all ? (int32_t)cap : all;
+}
+
+// What a decode call over n_seq rows needs of its workspace.
+size_t decode_ws_bytes(const Geo &g, const qwfn_qsa_shape *s, int32_t n_seq, int32_t max_seq_len) {
+    return ws_layout(g, n_seq, max_seq_len, max_selected(s, max_seq_len)).total;
+}
+
+// Whether n_pos chained positions can go out together: the attention selects
+// for itself, and the local window is long enough that a block a position
+// completes is in every later position's window, so no score needs its pooled
+// key within the call (it is pooled after the launches).
+bool chain_together(const Geo &g, const qwfn_qsa_shape *s, int32_t n_seq, int32_t n_pos, int32_t max_seq_len) {
+    return n_pos > 1 && g.local >= n_pos && attn_select_fits(g, n_seq, max_seq_len, max_selected(s, max_seq_len));
 }
 
 // Common checks of the per-call sequence arguments.
@@ -347,7 +360,10 @@ int qwfn_qsa_workspace_bytes(const qwfn_qsa_shape *shape, int32_t n_seq, int32_t
         return fail(QWFN_EINVAL, "workspace_bytes: bytes NULL or n_seq / max_seq_len < 1");
     if ((int64_t)n_seq * shape->n_head_kv > kMaxCounters)
         return fail(QWFN_ERANGE, "n_seq * n_head_kv exceeds %d", kMaxCounters);
-    *bytes = ws_layout(g, n_seq, max_seq_len, max_selected(shape, max_seq_len)).total;
+    // and, for a few sequences, the rows of a chained call's positions together
+    const int32_t rows = std::max(n_seq, std::min(n_seq * kMaxChain, kChainRows));
+    *bytes = std::max(decode_ws_bytes(g, shape, n_seq, max_seq_len),
+                      chain_together(g, shape, n_seq, 2, max_seq_len) ? decode_ws_bytes(g, shape, rows, max_seq_len) : 0);
     return ok();
 }
 
@@ -570,29 +586,54 @@ int qwfn_sparse_attn_decode_chain(const qwfn_qsa_shape *shape, const qwfn_kv_vie
     Ws w;
     if ((rc = bind_ws(g, n_seq, max_seq_len, msel, ws, ws_bytes, &w))) return rc;
     hipStream_t st = (hipStream_t)stream;
-    // position k's lengths: seq_len + k (the first position reads seq_len itself)
-    hipError_t e = n_pos > 1 ? launch_chain_lens(seq_len, n_seq, n_pos, w.lens, st) : hipSuccess;
-    if (e != hipSuccess) return hip_fail(e, "decode: chain lengths");
+    hipError_t e = hipSuccess;
     // one or a few sequences: the attention workgroups select for themselves
     // (no launch between the scores and the attention; at eight sequences a
     // selection launch of one workgroup per (sequence, KV head) before a
     // given-selection attention measured 29.4 against 26.9 us a step)
     const bool own = attn_select_fits(g, n_seq, max_seq_len, msel);
     const size_t row_b = (size_t)g.hd * (src_dtype == QWFN_SRC_F32 ? 4 : 2);
-    for (int32_t k = 0; k < n_pos; ++k) {
-        const int32_t *len_k = k == 0 ? seq_len : w.lens + (size_t)k * n_seq;
+    // The chain's positions as rows of one launch each of scoring (which appends
+    // every row first), attention and merge, as many as the workspace holds: a
+    // position's cells end at its own length, so it reads no later row.  Else one
+    // position after the other.  Four positions of one sequence at 32,771 tokens: 60.2
+    // -> 23.8 us.
+    int32_t group = 1;
+    if (chain_together(g, shape, n_seq, n_pos, max_seq_len))
+        for (group = n_pos; group > 1 && decode_ws_bytes(g, shape, group * n_seq, max_seq_len) > ws_bytes;) --group;
+    for (int32_t k = 0; k < n_pos; k += group) {
+        const int32_t np = std::min(group, n_pos - k), rows = np * n_seq;
+        const bool many = np > 1;
+        Geo gk = g;
+        if (many) {
+            gk.chain = n_seq;
+            if ((rc = bind_ws(g, rows, max_seq_len, msel, ws, ws_bytes, &w))) return rc;
+        } else if (group > 1) {
+            if ((rc = bind_ws(g, n_seq, max_seq_len, msel, ws, ws_bytes, &w))) return rc;
+        }
+        // position k's lengths: seq_len + k (the first position alone reads seq_len itself)
+        const int32_t *len_k = seq_len;
+        if (many || k > 0) {
+            e = launch_chain_lens(seq_len, n_seq, k, np, max_seq_len, w.lens, st);
+            if (e != hipSuccess) return hip_fail(e, "decode: chain lengths");
+            len_k = w.lens;
+        }
         const float *q_k = q + (size_t)k * n_seq * g.H * g.hd;
         const size_t kv_off = (size_t)k * n_seq * g.Hkv * row_b;
         const FusedAppend fa{(const uint8_t *)k_new + kv_off, (const uint8_t *)v_new + kv_off,
-                             src_dtype == QWFN_SRC_F16, 1};
+                             src_dtype == QWFN_SRC_F16, many ? 2 : 1};
         float *out_k = out + (size_t)k * n_seq * g.H * g.hd;
         int32_t *sel = sel_out ? sel_out + (size_t)k * n_seq * g.Hkv * msel : w.sel;
         int32_t *nsel = n_sel_out ? n_sel_out + (size_t)k * n_seq * g.Hkv : w.nsel;
-        e = launch_indexer(g, *view, q_k, len_k, n_seq, max_seq_len, sel, nsel, msel, w, fa, st, !own);
+        e = launch_indexer(gk, *view, q_k, len_k, rows, max_seq_len, sel, nsel, msel, w, fa, st, !own);
         if (e != hipSuccess) return hip_fail(e, "decode: indexer");
-        e = own ? launch_attention_select(g, *view, q_k, len_k, n_seq, max_seq_len, sel, nsel, msel, out_k, w, st)
-                : launch_attention(g, *view, q_k, len_k, n_seq, max_seq_len, sel, nsel, msel, out_k, w, st);
+        e = own ? launch_attention_select(gk, *view, q_k, len_k, rows, max_seq_len, sel, nsel, msel, out_k, w, st)
+                : launch_attention(gk, *view, q_k, len_k, rows, max_seq_len, sel, nsel, msel, out_k, w, st);
         if (e != hipSuccess) return hip_fail(e, "decode: attention");
+        if (many) {
+            e = launch_pool(gk, *view, nullptr, nullptr, rows, 0, 0, st, len_k);
+            if (e != hipSuccess) return hip_fail(e, "decode: pool");
+        }
     }
     return ok();
 }
@@ -653,6 +694,9 @@ int qwfn_sparse_attn_decode_noalloc(const qwfn_qsa_shape *shape, const qwfn_kv_v
     size_t need = 0;
     int rc = qwfn_qsa_workspace_bytes(shape, n_seq, max_seq_len, &need);
     if (rc) return rc;
+    Geo g;
+    if ((rc = make_geo(shape, nullptr, &g, false))) return rc;
+    need = decode_ws_bytes(g, shape, n_seq, max_seq_len);          // one position
     if (need > kScratchBytes)
         return fail(QWFN_ERANGE,
                     "decode_noalloc: n_seq %d at max_seq_len %d needs %zu bytes of workspace, more than the "

@@ -352,11 +352,12 @@ __device__ __forceinline__ void fused_append_pool(const Geo &g, const qwfn_kv_vi
     const int L = seq_len[s];
     if (L < 1 || L > max_seq_len) return;
     const int p = L - 1;
-    const int32_t pp = phys_page(g, v.page_table, s, p);
+    const int cs = cache_seq(g, s);
+    const int32_t pp = phys_page(g, v.page_table, cs, p);
     if (pp < 0) { if (tid == 0 && gh == 0) set_status(v.status, QWFN_STATUS_PAGE_RANGE); return; }
     const int row = p % g.pt;
     // a completed block's older members go to LDS while the new row is quantized
-    const bool complete = L % g.bt == 0;
+    const bool complete = fa.enabled == 1 && L % g.bt == 0;
     const bool early = complete && g.bt > 1 && g.bt - 1 <= stage_max_t<HD, KT>();
     const uint8_t *kpage = (const uint8_t *)v.k_pages + (int64_t)pp * g.page_bytes;
     if (early)
@@ -402,7 +403,7 @@ __device__ __forceinline__ void fused_append_pool(const Geo &g, const qwfn_kv_vi
     __syncthreads();
     if (!complete) return;                         // the block is not complete yet
     const int b = p / g.bt;
-    float *dst = v.pooled + (((int64_t)s * g.Hkv + gh) * g.bps + b) * HD;
+    float *dst = v.pooled + (((int64_t)cs * g.Hkv + gh) * g.bps + b) * HD;
     if (early) {
 #pragma clang fp contract(off)
         if (tid < HD)

@@ -824,7 +824,7 @@ k_dec(Geo g, qwfn_kv_view v, const float *__restrict__ q, const int32_t *__restr
     // prefill mode (gathered tiles): launch "sequence" s is query s of cache
     // sequence pf_seq, of length pf_pos0 + s + 1
     const int L = GATH ? seq_length(g, seq_len[g.pf ? 0 : s], s) : seq_len[s];
-    const int32_t *prow = v.page_table + (int64_t)(GATH ? cache_seq(g, s) : s) * g.pps;
+    const int32_t *prow = v.page_table + (int64_t)cache_seq(g, s) * g.pps;
     const int npt = min(g.pps, (max_seq_len + g.pt - 1) / g.pt);
     const bool park = (MODE != kDense || GATH) && npt <= kDecPtLds;
     constexpr int PTV = kDecPtLds / (4 * kDecThreads);   // 16-byte page-table loads a thread at most
@@ -1768,7 +1768,9 @@ void launch_dec_tm(const Geo &g, const qwfn_kv_view &v, const float *q, const in
 template <int HD, int G, int MODE, int KPT, bool RF, int LY>
 int launch_dec_t(const Geo &g, const qwfn_kv_view &v, const float *q, const int32_t *seq_len, int32_t n_seq,
                  int32_t max_seq_len, int32_t *sel, int32_t *nsel, int32_t max_sel, const Ws &ws, hipStream_t st) {
-    const int64_t pairs = (int64_t)n_seq * g.Hkv;
+    // (chained positions: the choice of a call of one position, so a position's
+    // result does not depend on how many go out together)
+    const int64_t pairs = (int64_t)(g.chain ? g.chain : n_seq) * g.Hkv;
     const int npt_lds = dec_npt_lds(g, max_seq_len, LY != kLyQ8 ? kGiven : MODE);
     const int d1 = dec_union_bytes<HD, G, MODE, 1, LY>() + 4 * npt_lds;
     const int d2 = dec_union_bytes<HD, G, MODE, 2, LY>() + 4 * npt_lds;

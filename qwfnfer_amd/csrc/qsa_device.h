@@ -50,8 +50,11 @@ __device__ __forceinline__ int64_t chunk_off(const Geo &g, int gh, int row, int 
 }
 
 // Cache sequence and length of launch sequence s (prefill: query s of one
-// cache sequence, see Geo::pf).  `raw` is seq_len[s] as loaded.
-__device__ __forceinline__ int cache_seq(const Geo &g, int s) { return g.pf ? g.pf_seq : s; }
+// cache sequence, see Geo::pf; chained positions: Geo::chain).  `raw` is
+// seq_len[s] as loaded.
+__device__ __forceinline__ int cache_seq(const Geo &g, int s) {
+    return g.pf ? g.pf_seq : g.chain > 1 ? s % g.chain : g.chain ? 0 : s;
+}
 __device__ __forceinline__ int seq_length(const Geo &g, int raw, int s) { return g.pf ? g.pf_pos0 + s + 1 : raw; }
 
 __device__ __forceinline__ int8_t to_i8(float r) {

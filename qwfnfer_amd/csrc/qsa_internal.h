@@ -35,6 +35,10 @@ struct Geo {
     // Prefill mode (pf = 1): "sequence" s of a launch is query s of cache
     // sequence pf_seq at position pf_pos0 + s, i.e. seq_len pf_pos0 + s + 1.
     int32_t pf, pf_seq, pf_pos0;
+    // Several chained decode positions in one launch (0: none): "sequence" s of
+    // the launch is a position of cache sequence s % chain, its length in the
+    // launch's length array.
+    int32_t chain;
 };
 
 // Device pointers into a caller workspace (see qwfn_qsa_workspace_bytes).
@@ -50,6 +54,7 @@ constexpr int32_t kIdxRegKeys = 8192;
 constexpr int32_t kCutKeys = 4096;
 constexpr int32_t kCutWgMax = 64;
 constexpr int32_t kMaxChain = 8;          // positions of one chained decode call (qwfn_sparse_attn_decode_chain)
+constexpr int32_t kChainRows = 16;        // (position, sequence) rows the decode workspace holds for it at least
 constexpr int32_t kScoreRecBlocks = 16;   // blocks per (min, max) score record of the fused call's scoring
 constexpr int32_t kIdxChunkBlocks = 64;   // blocks an indexer workgroup scores (its candidate slots)
 constexpr int32_t kIdxCutSamples = 1024;  // sampled scores of a long decode row's cut
@@ -83,7 +88,8 @@ WsLayout ws_layout(const Geo &g, int32_t n_seq, int32_t max_seq_len, int32_t max
                    bool cut = true);
 Ws ws_bind(void *base, const WsLayout &l);
 
-// Fused-append arguments of the decode step (enabled == 0: plain indexer).
+// Fused-append arguments of the decode step (enabled == 0: plain indexer; 2:
+// append only, the completed blocks are pooled by a launch of their own).
 struct FusedAppend {
     const void *k_new, *v_new;       // [n_seq][Hkv][hd]
     int32_t src_f16, enabled;
@@ -131,8 +137,10 @@ inline int32_t kv_row_bytes(int32_t kt, int32_t hd) {
 }
 
 hipError_t launch_fill_zero(void *p, size_t bytes, hipStream_t st);
-// lens[k][s] = seq_len[s] + k for k < n_pos (one small launch)
-hipError_t launch_chain_lens(const int32_t *seq_len, int32_t n_seq, int32_t n_pos, int32_t *lens, hipStream_t st);
+// lens[k][s] = seq_len[s] + pos0 + k for k < n_pos, 0 past max_seq_len (one
+// small launch)
+hipError_t launch_chain_lens(const int32_t *seq_len, int32_t n_seq, int32_t pos0, int32_t n_pos, int32_t max_seq_len,
+                             int32_t *lens, hipStream_t st);
 
 // The checkpoint's own indexer keys (qwfn_idx_shape): raw fp16 keys of `dim`
 // values per token, pooled per block with RMSNorm * k_norm, then the first nd
@@ -205,7 +213,7 @@ hipError_t launch_append(const Geo &g, const qwfn_kv_view &v, const void *k, con
                          int32_t n_rows, int32_t seq_const, int32_t pos0, hipStream_t st,
                          const int32_t *len = nullptr);
 // seq_ids NULL: every block in seq_const; block_ids NULL: blocks blk0 + [0, n_blocks);
-// len (decode): sequence i's block holding len[i] - 1 when that token completes it.
+// len (decode): sequence i's (with Geo::chain, position i's) block holding len[i] - 1 when that token completes it.
 hipError_t launch_pool(const Geo &g, const qwfn_kv_view &v, const int32_t *seq_ids,
                        const int32_t *block_ids, int32_t n_blocks, int32_t seq_const,
                        int32_t blk0, hipStream_t st, const int32_t *len = nullptr);

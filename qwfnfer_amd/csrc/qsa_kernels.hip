@@ -38,13 +38,17 @@ hipError_t launch_fill_zero(void *p, size_t bytes, hipStream_t st) {
     return hipGetLastError();
 }
 
-__global__ void k_chain_lens(const int32_t *__restrict__ seq_len, int32_t n_seq, int32_t n_pos,
-                             int32_t *__restrict__ lens) {
-    for (int i = (int)threadIdx.x; i < n_seq * n_pos; i += (int)blockDim.x) lens[i] = seq_len[i % n_seq] + i / n_seq;
+__global__ void k_chain_lens(const int32_t *__restrict__ seq_len, int32_t n_seq, int32_t pos0, int32_t n_pos,
+                             int32_t max_seq_len, int32_t *__restrict__ lens) {
+    for (int i = (int)threadIdx.x; i < n_seq * n_pos; i += (int)blockDim.x) {
+        const int64_t L = (int64_t)seq_len[i % n_seq] + pos0 + i / n_seq;
+        lens[i] = L <= max_seq_len ? (int32_t)max(L, (int64_t)0) : 0;   // 0: out of range
+    }
 }
 
-hipError_t launch_chain_lens(const int32_t *seq_len, int32_t n_seq, int32_t n_pos, int32_t *lens, hipStream_t st) {
-    hipLaunchKernelGGL(k_chain_lens, dim3(1), dim3(256), 0, st, seq_len, n_seq, n_pos, lens);
+hipError_t launch_chain_lens(const int32_t *seq_len, int32_t n_seq, int32_t pos0, int32_t n_pos, int32_t max_seq_len,
+                             int32_t *lens, hipStream_t st) {
+    hipLaunchKernelGGL(k_chain_lens, dim3(1), dim3(256), 0, st, seq_len, n_seq, pos0, n_pos, max_seq_len, lens);
     return hipGetLastError();
 }
 
@@ -94,7 +98,7 @@ k_pool(Geo g, qwfn_kv_view v, const int32_t *seq_ids, const int32_t *block_ids, 
     __shared__ uint16_t sc[kStageRows * (HD / 32)];
     const int bi = blockIdx.x, gh = blockIdx.y, tid = threadIdx.x;
     if (len && (len[bi] < 1 || len[bi] % g.bt)) return;   // no block completed (a bad length is the append's report)
-    const int seq = len ? bi : seq_ids ? seq_ids[bi] : seq_const;
+    const int seq = len ? cache_seq(g, bi) : seq_ids ? seq_ids[bi] : seq_const;
     const int b = len ? (len[bi] - 1) / g.bt : block_ids ? block_ids[bi] : blk0 + bi;
     const bool report = (gh == 0 && tid == 0);
     if (seq < 0 || seq >= g.n_seq_view) { if (report) set_status(v.status, QWFN_STATUS_SEQ_RANGE); return; }
@@ -638,7 +642,7 @@ k_score(Geo g, qwfn_kv_view v, const float *__restrict__ q, const int32_t *seq_l
     // ends before reading keys nothing uses
     const int L = seq_len[s];
     const bool ok = L >= 1 && L <= max_seq_len;
-    if (gridDim.z > 1) {                           // (uniform)
+    if (gridDim.z > 1 && g.chain != 1) {           // (uniform; one sequence's chained positions are as one)
         const Ranges r0 = qsa_ranges(g, L);
         const int ne0 = r0.e_hi - r0.e_lo;
         if (!(ok && g.topk > 0 && ne0 > eff_topk(g, r0) && c * BPW < ne0)) return;
@@ -652,7 +656,7 @@ k_score(Geo g, qwfn_kv_view v, const float *__restrict__ q, const int32_t *seq_l
     const int j = tid & 3, hh = (tid >> 2) & 1, bl = tid >> 3;
     const int bi = c * BPW + bl;
     const int bp = min(g.sink + bi, g.bps - 1);
-    const int64_t prow = (((int64_t)s * g.Hkv + gh) * g.bps + bp) * HD;
+    const int64_t prow = (((int64_t)cache_seq(g, s) * g.Hkv + gh) * g.bps + bp) * HD;
     float4 p4[HD / 16];
     if (g.pooled_f16) {
         const uint16_t *P = reinterpret_cast<const uint16_t *>(v.pooled) + prow;
@@ -3191,7 +3195,7 @@ hipError_t launch_attention(const Geo &g, const qwfn_kv_view &v, const float *q,
 constexpr int32_t kAttnSelSeqs = 8;
 
 bool attn_select_fits(const Geo &g, int32_t n_seq, int32_t max_seq_len, int32_t max_sel) {
-    if (g.shared || g.topk <= 0 || g.pf || n_seq > kAttnSelSeqs) return false;
+    if (g.shared || g.topk <= 0 || g.pf || (g.chain ? g.chain : n_seq) > kAttnSelSeqs) return false;
     if (dec_kernels_for(g))
         return dec_select_fits(g, max_seq_len, max_sel);
     if (max_sel > kAttnSelMax || max_seq_len / g.bt > kKeysMax) return false;

@@ -166,3 +166,46 @@ def test_chain_in_one_hipgraph():
         torch.cuda.synchronize()
         assert torch.equal(o2, ref)
     assert qsa.read_status(dev) == 0
+
+
+@pytest.mark.parametrize("cfg,lengths,n_pos,part", [
+    (BASELINE, [64 * 110 - 2], 8, 1),                # eight rows in one launch, a block completed inside
+    (BASELINE, [64 * 110 - 2], 8, 3),                # a workspace for fewer: groups of positions, the last one short
+    (BASELINE, [64 * 110 - 2], 5, 8),                # a workspace for one position
+    (BASELINE, [300, 64 * 90 - 1, 5000, 129], 7, 1),   # groups of 16 rows over four sequences
+    (Cfg(local_tokens=3), [64 * 90 - 2, 5000], 3, 1),  # the shortest window that lets three go out together
+    (Cfg(local_tokens=2), [64 * 90 - 2, 5000], 3, 1),  # and one too short: position by position
+    (Cfg(kv_type=1), [64 * 90 - 2, 5000], 4, 1), (Cfg(kv_type=2), [64 * 90 - 2, 5000], 4, 1),
+    (Cfg(n_head=4, block_tokens=4, page_tokens=64, top_k_blocks=5, local_tokens=9), [201, 90], 6, 1),
+])
+def test_chain_groups_equal_single_calls(cfg, lengths, n_pos, part):
+    """However many positions a launch takes (by the workspace and the window),
+    every position's output and selection and the caches equal single calls'; the
+    last position, past max_seq_len, gives zeros and its status bit and writes
+    nothing."""
+    print(f"chain groups: lengths {lengths}, n_pos {n_pos}, workspace / {part}", flush=True)
+    _, dev, _, q, kn, vn = _setup(cfg, lengths, n_pos, seed=31)
+    twin = _clone(dev)
+    n_seq = len(lengths)
+    c = cfg_of(cfg)
+    cur = torch.tensor(lengths, dtype=torch.int32, device="cuda") + 1
+    max_len = max(lengths) + n_pos - 1                    # the longest sequence's last position is out of range
+    ws = qsa.Workspace(c, n_seq, max_len, nbytes=-(-c.workspace_bytes(n_seq, max_len) // part // 256) * 256 + 65536)
+    msel = c.max_selected(max_len)
+    qd, knd, vnd = torch.from_numpy(q).cuda(), torch.from_numpy(kn).cuda(), torch.from_numpy(vn).cuda()
+    sel = torch.zeros((n_pos, n_seq, cfg.n_head_kv, msel), dtype=torch.int32, device="cuda")
+    nsel = torch.zeros((n_pos, n_seq, cfg.n_head_kv), dtype=torch.int32, device="cuda")
+    out = qsa.sparse_attn_decode_chain(dev, qd, knd, vnd, cur, max_len, ws, sel=sel, n_sel=nsel)
+    ws1 = qsa.Workspace(c, n_seq, max_len)
+    for k in range(n_pos):
+        s1, n1 = torch.zeros_like(sel[k]), torch.zeros_like(nsel[k])
+        o1 = qsa.sparse_attn_decode(twin, qd[k].contiguous(), knd[k].contiguous(), vnd[k].contiguous(),
+                                    (cur + k).contiguous(), max_len, ws1, sel=s1, n_sel=n1)
+        torch.cuda.synchronize()
+        assert torch.equal(o1, out[k]) and torch.equal(n1, nsel[k]), f"position {k}"
+        m = torch.arange(msel, device="cuda") < n1[..., None]
+        assert torch.equal(s1[m], sel[k][m]), f"position {k}"
+    assert not out[n_pos - 1, int(np.argmax(lengths))].any()
+    assert qsa.read_status(dev) == qsa.read_status(twin) != 0
+    for name in ("k_pages", "v_pages", "pooled"):
+        assert torch.equal(getattr(dev, name), getattr(twin, name)), name
