@@ -592,6 +592,13 @@ int qwfn_sparse_attn_decode_chain(const qwfn_qsa_shape *shape, const qwfn_kv_vie
     // selection launch of one workgroup per (sequence, KV head) before a
     // given-selection attention measured 29.4 against 26.9 us a step)
     const bool own = attn_select_fits(g, n_seq, max_seq_len, msel);
+    // more sequences: scores, then the selections in a launch of their own (one
+    // workgroup a (sequence, KV head), started by the stream, where the indexer's
+    // last workgroups waited for each row's arrivals first): 32 sequences of
+    // 1,000 .. 40,000 tokens 57.5 -> 38.0 us a step, k_indexer 28.1 -> k_score 6.9 +
+    // k_sel 4.7.  Lengths that keep every block have nothing to select, and the
+    // launch would cost 3.5 us of 29.7
+    const bool apart = !own && dec_sel_fits(g, max_seq_len, msel) && max_seq_len > all_kept_len(g);
     const size_t row_b = (size_t)g.hd * (src_dtype == QWFN_SRC_F32 ? 4 : 2);
     // The chain's positions as rows of one launch each of scoring (which appends
     // every row first), attention and merge, as many as the workspace holds: a
@@ -625,7 +632,8 @@ int qwfn_sparse_attn_decode_chain(const qwfn_qsa_shape *shape, const qwfn_kv_vie
         float *out_k = out + (size_t)k * n_seq * g.H * g.hd;
         int32_t *sel = sel_out ? sel_out + (size_t)k * n_seq * g.Hkv * msel : w.sel;
         int32_t *nsel = n_sel_out ? n_sel_out + (size_t)k * n_seq * g.Hkv : w.nsel;
-        e = launch_indexer(gk, *view, q_k, len_k, rows, max_seq_len, sel, nsel, msel, w, fa, st, !own);
+        e = launch_indexer(gk, *view, q_k, len_k, rows, max_seq_len, sel, nsel, msel, w, fa, st, !own && !apart);
+        if (e == hipSuccess && apart) e = launch_dec_sel(gk, len_k, rows, max_seq_len, sel, nsel, msel, w, st);
         if (e != hipSuccess) return hip_fail(e, "decode: indexer");
         e = own ? launch_attention_select(gk, *view, q_k, len_k, rows, max_seq_len, sel, nsel, msel, out_k, w, st)
                 : launch_attention(gk, *view, q_k, len_k, rows, max_seq_len, sel, nsel, msel, out_k, w, st);

@@ -1869,6 +1869,29 @@ hipError_t launch_dec_selbig_t(const Geo &g, const qwfn_kv_view &v, const float 
     return launch_merge(g, v, seq_len, n_seq, max_seq_len, nsel, max_sel, false, out, ws, 1, st);
 }
 
+// The selection of kSelect alone, a launch of one workgroup per (KV head,
+// sequence) between the scoring and an attention over a given selection
+// (launch_dec_sel).
+template <int KPT>
+__global__ void __launch_bounds__(kDecThreads)
+k_sel(Geo g, const int32_t *__restrict__ seq_len, int32_t max_seq_len, int32_t *__restrict__ sel,
+      int32_t *__restrict__ nsel, int32_t max_sel, Ws ws) {
+#pragma clang fp contract(off)
+    __shared__ DecShared<1> sh;
+    __shared__ DecSel ss;
+    const int gh = blockIdx.x, s = blockIdx.y, tid = threadIdx.x;
+    const int pair = s * g.Hkv + gh;
+    const int L = seq_len[s];
+    float sv[KPT];
+    float2 rec[dec_rpl<KPT>()];
+    dec_load_sel_inputs<KPT>(g, ws, pair, sv, rec);
+    dec_zero_hist(ss);
+    __syncthreads();
+    const int n = dec_choose<KPT>(g, ws, L, max_seq_len, max_sel, sv, rec, ss, sh);
+    for (int i = tid; i < n; i += kDecThreads) sel[(int64_t)pair * max_sel + i] = sh.sel[i];
+    if (tid == 0) nsel[pair] = n;
+}
+
 // The selection of kSelBig alone, for the test entry point: one workgroup a
 // sequence over its score row (rows of nb_cap), the selection written out.
 // The inputs the product path takes from the append and indexer launches are

@@ -120,6 +120,27 @@ hipError_t launch_test_select_big(const Geo &g, const float *scores, int32_t nb_
     return hipGetLastError();
 }
 
+bool dec_sel_fits(const Geo &g, int32_t max_seq_len, int32_t max_sel) {
+    return !g.pf && !g.shared && g.topk > 0 && max_sel <= kDecSelMax &&
+           max_seq_len / g.bt - (g.sink & ~3) <= 32 * kDecThreads;
+}
+
+hipError_t launch_dec_sel(const Geo &g, const int32_t *seq_len, int32_t n_seq, int32_t max_seq_len, int32_t *sel,
+                          int32_t *nsel, int32_t max_sel, const Ws &ws, hipStream_t st) {
+    if (!dec_sel_fits(g, max_seq_len, max_sel)) return hipErrorInvalidValue;
+    const int span = max_seq_len / g.bt - (g.sink & ~3);
+    const dim3 grid((unsigned)g.Hkv, (unsigned)n_seq), blk(kDecThreads);
+    if (span <= 4 * kDecThreads)
+        hipLaunchKernelGGL(k_sel<4>, grid, blk, 0, st, g, seq_len, max_seq_len, sel, nsel, max_sel, ws);
+    else if (span <= 8 * kDecThreads)
+        hipLaunchKernelGGL(k_sel<8>, grid, blk, 0, st, g, seq_len, max_seq_len, sel, nsel, max_sel, ws);
+    else if (span <= 16 * kDecThreads)
+        hipLaunchKernelGGL(k_sel<16>, grid, blk, 0, st, g, seq_len, max_seq_len, sel, nsel, max_sel, ws);
+    else
+        hipLaunchKernelGGL(k_sel<32>, grid, blk, 0, st, g, seq_len, max_seq_len, sel, nsel, max_sel, ws);
+    return hipGetLastError();
+}
+
 hipError_t launch_dec_attention(const Geo &g, const qwfn_kv_view &v, const float *q, const int32_t *seq_len,
                                 int32_t n_seq, int32_t max_seq_len, const int32_t *sel, const int32_t *nsel,
                                 int32_t max_sel, float *out, const Ws &ws, bool select, hipStream_t st) {

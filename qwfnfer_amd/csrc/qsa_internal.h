@@ -41,6 +41,14 @@ struct Geo {
     int32_t chain;
 };
 
+// Tokens up to which every block of a sequence is kept (topk > 0): while the
+// eligible ones are at most top_k, (L - local) / bt - sink <= top_k, or, when the
+// count includes the forced blocks, while it has at most top_k blocks in all.
+inline int64_t all_kept_len(const Geo &g) {
+    return g.keep_total ? (int64_t)g.topk * g.bt
+                        : (int64_t)g.local + (int64_t)g.bt * ((int64_t)g.topk + g.sink + 1) - 1;
+}
+
 // Device pointers into a caller workspace (see qwfn_qsa_workspace_bytes).
 // The counter region sits at a fixed offset with a fixed capacity so every
 // call layout agrees on it; all other regions are per-call scratch.
@@ -290,6 +298,12 @@ bool attn_select_fits(const Geo &g, int32_t n_seq, int32_t max_seq_len, int32_t 
 hipError_t launch_attention_select(const Geo &g, const qwfn_kv_view &v, const float *q, const int32_t *seq_len,
                                    int32_t n_seq, int32_t max_seq_len, int32_t *sel, int32_t *nsel,
                                    int32_t max_sel, float *out, const Ws &ws, hipStream_t st);
+// The selection of launch_attention_select as a launch of its own, from the
+// scores of a scores-only indexer launch: per-head selections of at most 8192
+// eligible blocks and 1024 selected.
+bool dec_sel_fits(const Geo &g, int32_t max_seq_len, int32_t max_sel);
+hipError_t launch_dec_sel(const Geo &g, const int32_t *seq_len, int32_t n_seq, int32_t max_seq_len, int32_t *sel,
+                          int32_t *nsel, int32_t max_sel, const Ws &ws, hipStream_t st);
 // Combine of the attention partials: og = sum_i w_i O_i / sum_i w_i l_i over
 // the parts of tg tiles each (dense: every block below the length).
 hipError_t launch_merge(const Geo &g, const qwfn_kv_view &v, const int32_t *seq_len, int32_t n_seq,

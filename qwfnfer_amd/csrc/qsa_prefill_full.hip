@@ -713,12 +713,7 @@ constexpr int64_t kFullPairs = 1024, kFullPairsK = 768;   // (query, KV head) pa
 int32_t pf_full_queries(const Geo &g, int32_t pos0, int32_t n_q) {
     const int ly = full_layout(g);
     if (ly < 0) return 0;
-    // every block is kept while the eligible ones are at most top_k: (L -
-    // local) / bt - sink <= top_k, or, when the count includes the forced
-    // blocks, while the sequence has at most top_k blocks in all
-    const int64_t most = g.topk <= 0      ? (int64_t)pos0 + n_q
-                         : g.keep_total ? (int64_t)g.topk * g.bt
-                                        : (int64_t)g.local + (int64_t)g.bt * ((int64_t)g.topk + g.sink + 1) - 1;
+    const int64_t most = g.topk <= 0 ? (int64_t)pos0 + n_q : all_kept_len(g);
     const int64_t n = std::max<int64_t>(0, std::min<int64_t>(n_q, most - pos0));
     return n * g.Hkv >= (ly == kPlQ8 ? kFullPairs : kFullPairsK) ? (int32_t)n : 0;
 }

@@ -144,3 +144,15 @@ def test_checkpoint_rule_decode_pools_before_scoring(mode):
     # 9598 + 2 = 64 * 150: sequence 1 completes block 149 at step 2.  Each
     # completed block is whole, hence eligible, at the step that completes it.
     decode_steps(CKPT_RULE, [64 * 300 - 3, 64 * 150 - 2], steps=4, seed=760, modes=[mode] * 4, reattend=True)
+
+
+@pytest.mark.parametrize("cfg, lengths", [
+    (BASELINE, [4735, 4736, 4800, 9000, 1, 64, 20001, 5000, 12345]),      # nine: the first count past the attention's own selection
+    (Cfg(kv_type=1), [9000, 30, 5001, 4736] * 3), (Cfg(kv_type=2, n_head=8), [9000, 30, 5001, 4736] * 3),
+    (Cfg(local_tokens=0, sink_blocks=0, topk_counts_forced=1), [64 * 90 - 1, 4096, 9000] * 3),
+    (Cfg(n_head=4, block_tokens=4, page_tokens=64, top_k_blocks=5, local_tokens=9), [90, 3000, 7, 17, 33, 900, 8, 64, 65, 1000]),
+])
+def test_many_sequences_select_apart(cfg, lengths):
+    """More sequences than the attention selects for itself: scores, a selection launch,
+    the attention over it; lengths on both sides of the one that keeps every block."""
+    decode_steps(cfg, lengths, 2, seed=len(lengths))
