@@ -1796,6 +1796,18 @@ int launch_dec_t(const Geo &g, const qwfn_kv_view &v, const float *q, const int3
     return 4;
 }
 
+// Whether a given-selection or dense q8_0 call goes to launch_dec_walk: when its
+// tiles, one a workgroup, are more than the device holds of k_dec at once.
+template <int HD, int G>
+bool dec_walk_pays(const Geo &g, int32_t n_seq, int32_t max_seq_len, bool given, const Ws &ws) {
+    const int npt_lds = dec_npt_lds(g, max_seq_len, given ? kGiven : kDense);
+    const int64_t r = given ? dec_resident<HD, G, kGiven, 4, 1, false, kLyQ8>(
+                                  dec_union_bytes<HD, G, kGiven, 1, kLyQ8>() + 4 * npt_lds)
+                            : dec_resident<HD, G, kDense, 4, 1, false, kLyQ8>(
+                                  dec_union_bytes<HD, G, kDense, 1, kLyQ8>() + 4 * npt_lds);
+    return r > 0 && (int64_t)(g.chain ? g.chain : n_seq) * g.Hkv * ws.n_tiles > r;
+}
+
 template <int HD, int G, bool RF, int LY>
 hipError_t launch_dec_shape(const Geo &g, const qwfn_kv_view &v, const float *q, const int32_t *seq_len,
                             int32_t n_seq, int32_t max_seq_len, const int32_t *sel, const int32_t *nsel,
@@ -1819,6 +1831,10 @@ hipError_t launch_dec_shape(const Geo &g, const qwfn_kv_view &v, const float *q,
             tpw = launch_dec_t<HD, G, kSelect, 32, RF, LY>(g, v, q, seq_len, n_seq, max_seq_len, sl, ns, max_sel, ws, st);
         else
             return hipErrorInvalidValue;
+    } else if (LY == kLyQ8 && !RF && dec_walk_fits(g) && dec_walk_pays<HD, G>(g, n_seq, max_seq_len, sel != nullptr, ws)) {
+        tpw = dec_walk_tiles(g, (int64_t)(g.chain ? g.chain : n_seq) * g.Hkv, ws.n_tiles);
+        const hipError_t e = launch_dec_walk(g, v, q, seq_len, n_seq, max_seq_len, sel, nsel, max_sel, ws, tpw, st);
+        if (e != hipSuccess) return e;
     } else if (sel) {
         tpw = launch_dec_t<HD, G, kGiven, 4, RF, LY>(g, v, q, seq_len, n_seq, max_seq_len, sl, ns, max_sel, ws, st);
     } else {

@@ -289,6 +289,15 @@ hipError_t launch_prefill_attention(const Geo &g, const qwfn_kv_view &v, const f
 int32_t pf_full_queries(const Geo &g, int32_t pos0, int32_t n_q);
 hipError_t launch_prefill_full(const Geo &g, const qwfn_kv_view &v, const float *q, int32_t n_q, const float *vmax,
                                float *out, hipStream_t st);
+// Batched decode attention over a given selection (or every block, sel NULL) with
+// the prefill attention's wave walking the tiles: parts of tpw tiles
+// (dec_walk_tiles) a workgroup, partials in ws for launch_merge.  Fits: q8_0 in whole tiles, some head
+// shapes.
+bool dec_walk_fits(const Geo &g);
+int dec_walk_tiles(const Geo &g, int64_t pairs, int n_tiles);
+hipError_t launch_dec_walk(const Geo &g, const qwfn_kv_view &v, const float *q, const int32_t *seq_len, int32_t n_seq,
+                           int32_t max_seq_len, const int32_t *sel, const int32_t *nsel, int32_t max_sel,
+                           const Ws &ws, int32_t tpw, hipStream_t st);
 // Decode attention that makes its own selection from the scores of a
 // scores-only indexer launch, writing it to sel / nsel (the q8_0 matrix-core
 // kernel for its shapes, the general kernel for the other element types and

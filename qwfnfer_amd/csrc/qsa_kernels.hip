@@ -2645,32 +2645,49 @@ struct PfAttnLds {
 // Cells past the query's position have weight 0 and their V scale masked.
 // K and V tiles are addressed from a wave-uniform base plus a fixed per-lane
 // offset (no per-lane 64-bit address arithmetic per tile).
-// SPLIT (few pairs): `split` waves of the workgroup share a pair, wave u of
-// them taking tiles u, u + split, ..., and add up their states through LDS at
+// MODE kPfSplit (few pairs): `split` waves of the workgroup share a pair, wave u
+// of them taking tiles u, u + split, ..., and add up their states through LDS at
 // the end (pf_split picks the count).
-template <int HD, int G, bool SPLIT>
-__global__ void __launch_bounds__((PfAttnCfg<HD, G>::WAVES * 64))
+// MODE kPfDecode: a batched decode's attention over a given selection (sel) or
+// every block (sel NULL): grid (parts, Hkv, n_seq), kPfDecWaves waves a workgroup,
+// two workgroups a CU; the waves share tiles [part split, (part + 1) split) of a
+// (sequence, KV head) and leave one partial (max, sum, unnormalised O) for k_merge.
+// There 2^k follows the largest V scale of the tiles a wave has met (a power of
+// two, so O moves exactly when it changes).
+enum PfMode { kPfWhole = 0, kPfSplit = 1, kPfDecode = 2 };
+constexpr int kPfDecWaves = 4;
+template <int HD, int G, int MODE>
+constexpr int pf_waves() { return MODE == kPfDecode ? kPfDecWaves : PfAttnCfg<HD, G>::WAVES; }
+template <int HD, int G, int MODE>
+__global__ void __launch_bounds__((pf_waves<HD, G, MODE>() * 64), (MODE == kPfDecode ? 2 : 1))
 k_pf_attn(Geo g, qwfn_kv_view v, const float *__restrict__ q, int32_t n_q, const int32_t *__restrict__ sel,
           const int32_t *__restrict__ nsel, int32_t max_sel, const float *__restrict__ vmax,
-          float *__restrict__ out, int32_t split) {
+          float *__restrict__ out, int32_t split, const int32_t *__restrict__ seq_len, Ws ws) {
     using C = PfAttnCfg<HD, G>;
+    constexpr bool SPLIT = MODE != kPfWhole, DEC = MODE == kPfDecode;
+    constexpr int WAVES = pf_waves<HD, G, MODE>();
     constexpr int NJ = HD / 32, ND = HD / 16, NK4 = C::NK4, NS4 = C::NS4;
     static_assert(G <= 16, "one MFMA output column per query head");
-    __shared__ PfAttnLds<HD, G> shw[C::WAVES];
+    __shared__ PfAttnLds<HD, G> shw[WAVES];
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = threadIdx.x & 63;
-    const int nsp = SPLIT ? split : 1;               // waves a pair (divides WAVES)
+    const int nsp = DEC ? WAVES : SPLIT ? split : 1; // waves a pair (divides WAVES)
     const int sub = SPLIT ? wv % nsp : 0;            // this wave's place among them
-    int pair = SPLIT ? (int)blockIdx.x * (C::WAVES / nsp) + wv / nsp : (int)blockIdx.x * C::WAVES + wv;
-    const bool live = pair < n_q * g.Hkv;
+    int pair = DEC     ? (int)blockIdx.z * g.Hkv + (int)blockIdx.y
+               : SPLIT ? (int)blockIdx.x * (WAVES / nsp) + wv / nsp
+                       : (int)blockIdx.x * WAVES + wv;
+    const bool live = DEC || pair < n_q * g.Hkv;
     if (!SPLIT && !live) return;                     // a whole wave; no workgroup barrier follows
     if (SPLIT && !live) pair = n_q * g.Hkv - 1;      // (walks no tile and writes nothing)
     PfAttnLds<HD, G> &W = shw[wv];
     const int s = pair / g.Hkv, gh = pair - s * g.Hkv;
-    const int L = g.pf_pos0 + s + 1;
+    // (decode: n_q is the bound on the lengths; one out of range has no tile)
+    const int L = DEC ? seq_len[s] : g.pf_pos0 + s + 1;
     const int hn = l & 15, lg = l >> 4;              // MFMA column (head) and k-group of this lane
     const bool hv = hn < G;
-    const int n = min(nsel[pair], max_sel);
     const int tpb = g.bt / 64;
+    const int n = DEC && !(L >= 1 && L <= n_q) ? 0 : min(DEC && !sel ? (L - 1) / g.bt + 1 : nsel[pair], max_sel);
+    const int t_first = DEC ? (int)blockIdx.x * split : 0;           // this workgroup's tiles
+    if (DEC && t_first >= n * tpb) return;           // (the whole workgroup) no partial: the merge reads fewer
     const int32_t *selp = sel + (int64_t)pair * max_sel;
     // PAIR (8 heads, head_dim >= 128): QK's 16 columns hold every head twice,
     // columns h + 8 jp taking q8_0 blocks jj + jp NJ/2 -- so a lane's key
@@ -2738,20 +2755,21 @@ k_pf_attn(Geo g, qwfn_kv_view v, const float *__restrict__ q, int32_t n_q, const
     // p * dv * 2^kup stays below the fp16 maximum and its low half normal
     float kup;
     {
-        float dvm = vmax[gh * kVmaxWg + l % kVmaxWg];
+        float dvm = DEC ? 0.0f : vmax[gh * kVmaxWg + l % kVmaxWg];
         dvm = wave_max(dvm);
         int e2 = 0;
         frexpf(dvm, &e2);
         kup = dvm > 0.0f ? (float)(15 - e2) : 0.0f;
     }
+    if constexpr (DEC) kup = 60.0f;                  // no V scale met yet
     f4v o[ND];
 #pragma unroll
     for (int d = 0; d < ND; ++d) o[d] = f4v{0.0f, 0.0f, 0.0f, 0.0f};
     // running max starts at a finite floor far below any score, so exp2 of
     // (score - max) never sees inf - inf
     float m = -1e30f, lsum = 0.0f;                   // lsum in units of 2^kup
-    // this wave's tiles: tile sub + nsp t of the pair is its tile t
-    const int all_tiles = live ? n * tpb : 0;
+    // this wave's tiles: tile sub + nsp t of the pair (or its part) is its tile t
+    const int all_tiles = DEC ? min(split, n * tpb - t_first) : live ? n * tpb : 0;
     const int n_tiles = SPLIT ? (max(all_tiles - sub, 0) + nsp - 1) / nsp : all_tiles;
     // lane l's 16 bytes of a V tile's 1 KB transfer: dim row l / 4, quarter
     // (l % 4) ^ (row / 4 % 4)
@@ -2762,11 +2780,11 @@ k_pf_attn(Geo g, qwfn_kv_view v, const float *__restrict__ q, int32_t n_q, const
         int pg_l = 0, r0_l = 0, nv_l = 0;
         {
             if (tc + l < n_tiles) {
-                const int t = SPLIT ? sub + nsp * (tc + l) : tc + l;
-                const int blk = selp[t / tpb];
+                const int t = DEC ? t_first + sub + nsp * (tc + l) : SPLIT ? sub + nsp * (tc + l) : tc + l;
+                const int blk = DEC && !sel ? t / tpb : selp[t / tpb];
                 const int64_t t0 = (int64_t)blk * g.bt + (t % tpb) * 64;
                 if (blk >= 0 && t0 < L) {
-                    const int32_t pg = phys_page(g, v.page_table, g.pf_seq, (int)t0);
+                    const int32_t pg = phys_page(g, v.page_table, DEC ? cache_seq(g, s) : g.pf_seq, (int)t0);
                     if (pg >= 0) {
                         pg_l = pg;
                         r0_l = (int)(t0 % g.pt);
@@ -2898,6 +2916,24 @@ k_pf_attn(Geo g, qwfn_kv_view v, const float *__restrict__ q, int32_t n_q, const
                 for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
                     for (int w = 0; w < NJ; ++w) dvw[ks][w] = wvs[(32 * ks + 8 * lg) * NJ / 8 + w];
+                float kup_new = kup;
+                if constexpr (DEC) {
+                    // lane l: the largest finite scale of cell l (none past the query)
+                    float dvm = 0.0f;
+#pragma unroll
+                    for (int w = 0; w < NJ / 2; ++w) {
+                        const uint32_t x = reinterpret_cast<const uint32_t *>(wvs)[l * (NJ / 2) + w];
+#pragma unroll
+                        for (int e = 0; e < 2; ++e) {
+                            const uint32_t h = (e ? x >> 16 : x) & 0x7fffu;
+                            dvm = fmaxf(dvm, h < 0x7c00u && l < nv ? h2f((uint16_t)h) : 0.0f);
+                        }
+                    }
+                    dvm = wave_max(dvm);
+                    int e2 = 0;
+                    frexpf(dvm, &e2);
+                    if (dvm > 0.0f) kup_new = fminf(kup, (float)(15 - e2));
+                }
                 // the K chunks and scale rows are consumed: the next tile's may land
                 asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
                 if (ti + 1 < t_end) issue_k(ti + 1);
@@ -2927,7 +2963,8 @@ k_pf_attn(Geo g, qwfn_kv_view v, const float *__restrict__ q, int32_t n_q, const
                 if constexpr (PAIR) tm = fmaxf(tm, dppf<kDppRowRor8>(0.0f, tm));
                 tm *= lscale;                        // lscale > 0: the max commutes
                 const float m_new = fmaxf(m, tm);
-                const float alpha = __builtin_amdgcn_exp2f(m - m_new);
+                const float alpha = __builtin_amdgcn_exp2f(DEC ? (m - m_new) + (kup_new - kup) : m - m_new);
+                kup = kup_new;
                 const float bias = kup - m_new;
                 float tsum = 0.0f;
 #pragma unroll
@@ -3037,13 +3074,13 @@ k_pf_attn(Geo g, qwfn_kv_view v, const float *__restrict__ q, int32_t n_q, const
         const int w0 = wv - sub;
         if (hv && lg == 0) {
             W.p[hn][0] = m;
-            W.p[hn][1] = lsum;
+            W.p[hn][1] = DEC ? ldexpf(lsum, -(int)kup) : lsum;       // (O and the sum carry the wave's 2^k)
         }
         __syncthreads();
         if (hv) {
             float mx = m;
             for (int u = 0; u < nsp; ++u) mx = fmaxf(mx, shw[w0 + u].p[hn][0]);
-            const float wt = __builtin_amdgcn_exp2f(m - mx);
+            const float wt = __builtin_amdgcn_exp2f(DEC ? (m - mx) - kup : m - mx);
             float *ow = reinterpret_cast<float *>(&W.buf[0]) + hn * HD;
 #pragma unroll
             for (int d = 0; d < ND; ++d)
@@ -3060,6 +3097,12 @@ k_pf_attn(Geo g, qwfn_kv_view v, const float *__restrict__ q, int32_t n_q, const
             for (int u = 0; u < nsp; ++u) {
                 ls = __builtin_fmaf(shw[w0 + u].p[h][1], __builtin_amdgcn_exp2f(shw[w0 + u].p[h][0] - mx), ls);
                 t += reinterpret_cast<const f4v *>(&shw[w0 + u].buf[0])[i];
+            }
+            if constexpr (DEC) {
+                const int64_t pb = ((int64_t)pair * ws.n_tiles + blockIdx.x) * G;
+                reinterpret_cast<f4v *>(ws.part_o + pb * HD)[i] = t;
+                if (i % (HD / 4) == 0) *reinterpret_cast<float2 *>(&ws.part_ml[(pb + h) * 2]) = make_float2(mx, ls);
+                continue;
             }
             const float inv = ls > 0.0f ? 1.0f / ls : 0.0f;
             reinterpret_cast<f4v *>(out + ((int64_t)s * g.H + gh * G) * HD)[i] = t * inv;
@@ -3122,11 +3165,48 @@ static void launch_pf_attn_t(const Geo &g, const qwfn_kv_view &v, const float *q
     const int split = pf_split((int64_t)n_call * g.Hkv, WAVES, max_sel * (g.bt / 64));
     const dim3 grid((unsigned)((pairs * split + WAVES - 1) / WAVES));
     if (split == 1)
-        hipLaunchKernelGGL((k_pf_attn<HD, G, false>), grid, dim3(WAVES * 64), 0, st, g, v, q, n_q, sel, nsel, max_sel,
-                           vmax, out, 1);
+        hipLaunchKernelGGL((k_pf_attn<HD, G, kPfWhole>), grid, dim3(WAVES * 64), 0, st, g, v, q, n_q, sel, nsel, max_sel,
+                           vmax, out, 1, nullptr, Ws{});
     else
-        hipLaunchKernelGGL((k_pf_attn<HD, G, true>), grid, dim3(WAVES * 64), 0, st, g, v, q, n_q, sel, nsel, max_sel,
-                           vmax, out, split);
+        hipLaunchKernelGGL((k_pf_attn<HD, G, kPfSplit>), grid, dim3(WAVES * 64), 0, st, g, v, q, n_q, sel, nsel, max_sel,
+                           vmax, out, split, nullptr, Ws{});
+}
+
+// One tile a wave while the call's tiles (at most) are under two rounds of the device's
+// waves, else two, and at most 96 parts a row, which the merge reads on a workgroup
+// a head.  Measured, us a step (k_dec; parts of 4, by this rule, of 12 tiles): 32
+// sequences of 1,000 .. 40,000 tokens 39.8; 39.8, 39.2, 40.2 (35.5 by the rule in another
+// run), 32 of 40,000 49.1; 50.8, 50.7, 46.5, 16 of 1,000 .. 160,000 30.1; 30.5, 30.5, 32.6;
+// dense, 32 of 1,000 .. 16,000 61.3; 52.6, 47.3, 43.9, 16 of 16,000 55.1; 54.7, 47.6, 46.9,
+// 16 of 1,000 .. 16,000 37.0; 32.0, 30.7, 33.0, one of 100,000 43.4; 30.7, 30.6, 30.4 (of 4
+// tiles without the bound 43.4).
+int dec_walk_tiles(const Geo &g, int64_t pairs, int n_tiles) {
+    const int64_t waves = 2 * (int64_t)device_cus() * kPfDecWaves;
+    const int64_t per = std::min<int64_t>(2, pairs * n_tiles / waves);
+    const int64_t most = (n_tiles + 96 * kPfDecWaves - 1) / (96 * kPfDecWaves);
+    return (int)std::max<int64_t>(std::max<int64_t>(1, per), most) * kPfDecWaves;
+}
+
+hipError_t launch_dec_walk(const Geo &g, const qwfn_kv_view &v, const float *q, const int32_t *seq_len, int32_t n_seq,
+                           int32_t max_seq_len, const int32_t *sel, const int32_t *nsel, int32_t max_sel,
+                           const Ws &ws, int32_t tpw, hipStream_t st) {
+    // an odd count of parts: workgroups go to the eight XCDs in turn, and the first parts
+    // of short rows would otherwise meet on the same ones (dense, 32 sequences of 1,000
+    // .. 16,000 tokens: 69.5 us with 32 parts, 47.3 with 33)
+    const dim3 grid((unsigned)((ws.n_tiles + tpw - 1) / tpw) | 1u, (unsigned)g.Hkv, (unsigned)n_seq);
+#define X(HD_, G_)                                                                                                  \
+    if (g.hd == HD_ && g.G == G_) {                                                                                 \
+        QWFN_LAUNCH(kTimedAttention, (k_pf_attn<HD_, G_, kPfDecode>), grid, dim3(kPfDecWaves * 64), st, g, v, q,     \
+                    max_seq_len, sel, nsel, max_sel, nullptr, nullptr, tpw, seq_len, ws);                           \
+        return hipGetLastError();                                                                                   \
+    }
+    X(128, 8) X(128, 4) X(64, 8)
+#undef X
+    return hipErrorInvalidValue;
+}
+
+bool dec_walk_fits(const Geo &g) {
+    return g.vdim && !g.pf && !g.round_f16 && ((g.hd == 128 && (g.G == 8 || g.G == 4)) || (g.hd == 64 && g.G == 8));
 }
 
 hipError_t launch_prefill_attention(const Geo &g, const qwfn_kv_view &v, const float *q, int32_t n_q, int32_t n_call,

@@ -156,3 +156,40 @@ def test_many_sequences_select_apart(cfg, lengths):
     """More sequences than the attention selects for itself: scores, a selection launch,
     the attention over it; lengths on both sides of the one that keeps every block."""
     decode_steps(cfg, lengths, 2, seed=len(lengths))
+
+
+@pytest.mark.parametrize("cfg, lengths", [
+    (BASELINE, [4736 + 130 * i + 7 * i * i for i in range(10)] + [1, 63, 64, 65, 600, 30000]),
+    (Cfg(n_head=8), [5000 + 211 * i for i in range(16)]), (Cfg(head_dim=64), [5000 + 211 * i for i in range(24)]),
+    (Cfg(block_tokens=128, top_k_blocks=32), [4500 + 333 * i for i in range(16)]),
+    (Cfg(top_k_blocks=0), [20001, 1, 64, 9999, 5000, 20000, 17, 640]), (Cfg(top_k_blocks=0), [60001, 50000]),
+])
+def test_batched_attention_walks_tiles(cfg, lengths):
+    """Batches of more tiles than the device holds one a workgroup: the waves of a
+    workgroup share a part of a sequence's tiles (one, two or more a wave, parts that end
+    inside it, empty ones past a short sequence)."""
+    decode_steps(cfg, lengths, 1, seed=len(lengths), reattend=True)
+
+
+def test_batched_attention_wide_v_scales():
+    """V blocks over six decades of scale, the largest in any tile of a wave's:
+    its weight scale follows the largest met."""
+    cfg = Cfg(top_k_blocks=0)
+    rng = np.random.default_rng(3)
+    L = 70000
+    dev, host = make_pair(cfg, 1, L // cfg.page_tokens + 1)
+
+    def rows(rng, n, cfg):
+        k, v = kv_rows(rng, n, cfg, scaled=False)
+        v *= np.exp(rng.uniform(np.log(1e-3), np.log(1e3), (n // 64 + 1, 1, 1))).astype(np.float32).repeat(64, 0)[:n]
+        return k, v
+
+    fill(dev, host, rng, [L], rows=rows)
+    q = rng.standard_normal((1, cfg.n_head, cfg.head_dim), dtype=np.float32)
+    c = cfg_of(cfg)
+    out = qsa.sparse_decode_attn(dev, torch.from_numpy(q).cuda(), torch.tensor([L], dtype=torch.int32, device="cuda"), L,
+                                 qsa.Workspace(c, 1, L))
+    nb = (L + 63) // 64
+    sel = np.broadcast_to(np.arange(nb, dtype=np.int32), (1, cfg.n_head_kv, nb)).copy()
+    ref = host.attention_f64(q, np.array([L], np.int32), sel, np.full((1, cfg.n_head_kv), nb, np.int32))
+    assert_close_attn(np_of(out), ref)
