@@ -115,13 +115,20 @@ def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
 
 def _stream(stream) -> int:
     if stream is None:
-        return torch.cuda.current_stream().cuda_stream
+        if not torch.cuda.is_initialized():
+            return torch.cuda.current_stream().cuda_stream
+        # the same handle without the Stream object
+        return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
     if isinstance(stream, torch.cuda.Stream):
         return stream.cuda_stream
     return int(stream)
 
 
 def _need(t: torch.Tensor, name: str, dtype: torch.dtype, numel: Optional[int] = None) -> None:
+    # the usual case in one expression; what fails it is told apart below
+    if (isinstance(t, torch.Tensor) and t.is_cuda and t.dtype is dtype and t.is_contiguous() and
+            (numel is None or t.numel() == numel)):
+        return
     if not isinstance(t, torch.Tensor):
         raise TypeError(f"{name} must be a torch.Tensor")
     if t.device.type != "cuda":
@@ -151,6 +158,8 @@ class KvCache:
     page_table: torch.Tensor
     status: torch.Tensor
     _view: KvView = field(default=None, repr=False)
+    _shape: tuple = field(default=None, repr=False, compare=False)
+    _msel: tuple = field(default=None, repr=False, compare=False)
 
     @classmethod
     def allocate(cls, cfg: QsaConfig, n_seq: int, pages_per_seq: int,
@@ -189,6 +198,22 @@ class KvCache:
     @property
     def n_phys_pages(self) -> int:
         return self.k_pages.numel() // self.cfg.page_bytes()
+
+    # The C struct of cfg, and its last max_selected, kept between calls (a decode call's
+    # host time: each fills fourteen fields through ctypes; at 4,096 tokens the host and
+    # not the GPU paces the calls, 18.8 us a call before and 14.6 now).  A configuration
+    # is frozen, and the tuple holds it, so the same object means the same values.
+    def c_shape(self) -> QsaShape:
+        got = self._shape
+        if got is None or got[0] is not self.cfg:
+            got = self._shape = (self.cfg, self.cfg.shape())
+        return got[1]
+
+    def max_selected(self, max_seq_len: int) -> int:
+        got = self._msel
+        if got is None or got[0] is not self.cfg or got[1] != max_seq_len:
+            got = self._msel = (self.cfg, max_seq_len, self.cfg.max_selected(max_seq_len))
+        return got[2]
 
     def view(self) -> KvView:
         if self._view is None:
@@ -269,7 +294,7 @@ def append_q8_0(cache: KvCache, k: torch.Tensor, v: torch.Tensor, pos: torch.Ten
     _need(pos, "pos", torch.int32)
     if seq_ids is not None:
         _need(seq_ids, "seq_ids", torch.int32, n_rows)
-    s = cfg.shape()
+    s = cache.c_shape()
     call("qwfn_kv_append_q8_0", C.byref(s), C.byref(cache.view()), k.data_ptr(), v.data_ptr(),
          _lib.SRC_F16 if k.dtype == torch.float16 else _lib.SRC_F32, _ptr(seq_ids), pos.data_ptr(),
          n_rows, _stream(stream))
@@ -281,7 +306,7 @@ def pool_update(cache: KvCache, block_ids: torch.Tensor, seq_ids: Optional[torch
     _need(block_ids, "block_ids", torch.int32)
     if seq_ids is not None:
         _need(seq_ids, "seq_ids", torch.int32, block_ids.numel())
-    s = cache.cfg.shape()
+    s = cache.c_shape()
     call("qwfn_pool_update", C.byref(s), C.byref(cache.view()), _ptr(seq_ids), block_ids.data_ptr(),
          block_ids.numel(), _stream(stream))
 
@@ -289,7 +314,7 @@ def pool_update(cache: KvCache, block_ids: torch.Tensor, seq_ids: Optional[torch
 def pool_rebuild(cache: KvCache, seq: int, n_whole: int, stream=None) -> None:
     """qsa_pool_rebuild after a prefill: pool blocks [0, n_whole) of ``seq``
     (src/qwfn_graph.cpp:431-448, src/qwfn_engine.cpp:761-798)."""
-    s = cache.cfg.shape()
+    s = cache.c_shape()
     call("qwfn_pool_rebuild", C.byref(s), C.byref(cache.view()), seq, n_whole, _stream(stream))
 
 
@@ -304,7 +329,7 @@ def export_rows_q8_0(cache: KvCache, seq: int, pos0: int, n_tokens: int, k: bool
     dev = cache.k_pages.device
     kr = torch.empty((n_tokens, rb), dtype=torch.uint8, device=dev) if k else None
     vr = torch.empty((n_tokens, rb), dtype=torch.uint8, device=dev) if v else None
-    s = cfg.shape()
+    s = cache.c_shape()
     call("qwfn_kv_export_q8_0", C.byref(s), C.byref(cache.view()), seq, pos0, n_tokens, _ptr(kr), _ptr(vr),
          _stream(stream))
     return kr, vr
@@ -325,7 +350,7 @@ def import_rows_q8_0(cache: KvCache, seq: int, pos0: int, k_rows: Optional[torch
     for t, name in ((k_rows, "k_rows"), (v_rows, "v_rows")):
         if t is not None:
             _need(t, name, torch.uint8, n_tokens * rb)
-    s = cfg.shape()
+    s = cache.c_shape()
     call("qwfn_kv_import_q8_0", C.byref(s), C.byref(cache.view()), seq, pos0, n_tokens, _ptr(k_rows),
          _ptr(v_rows), _stream(stream))
 
@@ -339,14 +364,14 @@ def indexer_topk(cache: KvCache, q: torch.Tensor, seq_len: torch.Tensor, max_seq
     n_seq = seq_len.numel()
     _need(q, "q", torch.float32, n_seq * cfg.n_head * cfg.head_dim)
     _need(seq_len, "seq_len", torch.int32)
-    max_sel = cfg.max_selected(max_seq_len)
+    max_sel = cache.max_selected(max_seq_len)
     if sel is None:
         sel = torch.empty((n_seq, cfg.n_head_kv, max_sel), dtype=torch.int32, device=q.device)
     if n_sel is None:
         n_sel = torch.empty((n_seq, cfg.n_head_kv), dtype=torch.int32, device=q.device)
     _need(sel, "sel", torch.int32)
     _need(n_sel, "n_sel", torch.int32, n_seq * cfg.n_head_kv)
-    s = cfg.shape()
+    s = cache.c_shape()
     call("qwfn_indexer_topk", C.byref(s), C.byref(cache.view()), q.data_ptr(), seq_len.data_ptr(), n_seq,
          max_seq_len, sel.data_ptr(), n_sel.data_ptr(), sel.shape[-1], ws.ptr(), ws.nbytes, _stream(stream))
     return sel, n_sel
@@ -363,7 +388,7 @@ def gather_dequant(cache: KvCache, seq_len: torch.Tensor, sel: Optional[torch.Te
     k = torch.empty((n_seq, cfg.n_head_kv, nc, cfg.head_dim), dtype=torch.float32, device=dev)
     v = torch.empty_like(k)
     cells = torch.empty((n_seq, cfg.n_head_kv, nc), dtype=torch.int32, device=dev)
-    s = cfg.shape()
+    s = cache.c_shape()
     call("qwfn_gather_dequant", C.byref(s), C.byref(cache.view()), seq_len.data_ptr(), n_seq, _ptr(sel),
          _ptr(n_sel), max_sel, k.data_ptr(), v.data_ptr(), cells.data_ptr(), _stream(stream))
     return k, v, cells
@@ -382,7 +407,7 @@ def sparse_decode_attn(cache: KvCache, q: torch.Tensor, seq_len: torch.Tensor, m
         out = torch.empty((n_seq, cfg.n_head, cfg.head_dim), dtype=torch.float32, device=q.device)
     _need(out, "out", torch.float32, n_seq * cfg.n_head * cfg.head_dim)
     max_sel = sel.shape[-1] if sel is not None else 0
-    s = cfg.shape()
+    s = cache.c_shape()
     call("qwfn_sparse_decode_attn", C.byref(s), C.byref(cache.view()), q.data_ptr(), seq_len.data_ptr(),
          n_seq, max_seq_len, _ptr(sel), _ptr(n_sel), max_sel, out.data_ptr(), ws.ptr(), ws.nbytes,
          _stream(stream))
@@ -410,9 +435,9 @@ def sparse_attn_decode(cache: KvCache, q: torch.Tensor, k_new: torch.Tensor, v_n
     if (sel is None) != (n_sel is None):
         raise ValueError("pass both sel and n_sel or neither")
     if sel is not None:                            # the kernels write max_selected entries a (sequence, KV head)
-        _need(sel, "sel", torch.int32, n_seq * cfg.n_head_kv * cfg.max_selected(max_seq_len))
+        _need(sel, "sel", torch.int32, n_seq * cfg.n_head_kv * cache.max_selected(max_seq_len))
         _need(n_sel, "n_sel", torch.int32, n_seq * cfg.n_head_kv)
-    s = cfg.shape()
+    s = cache.c_shape()
     call("qwfn_sparse_attn_decode", C.byref(s), C.byref(cache.view()), q.data_ptr(), k_new.data_ptr(),
          v_new.data_ptr(), _lib.SRC_F16 if k_new.dtype == torch.float16 else _lib.SRC_F32,
          seq_len.data_ptr(), n_seq, max_seq_len, out.data_ptr(), _ptr(sel), _ptr(n_sel), ws.ptr(),
@@ -448,9 +473,9 @@ def sparse_attn_decode_chain(cache: KvCache, q: torch.Tensor, k_new: torch.Tenso
     if (sel is None) != (n_sel is None):
         raise ValueError("pass both sel and n_sel or neither")
     if sel is not None:
-        _need(sel, "sel", torch.int32, n_pos * n_seq * cfg.n_head_kv * cfg.max_selected(max_seq_len))
+        _need(sel, "sel", torch.int32, n_pos * n_seq * cfg.n_head_kv * cache.max_selected(max_seq_len))
         _need(n_sel, "n_sel", torch.int32, n_pos * n_seq * cfg.n_head_kv)
-    s = cfg.shape()
+    s = cache.c_shape()
     call("qwfn_sparse_attn_decode_chain", C.byref(s), C.byref(cache.view()), q.data_ptr(), k_new.data_ptr(),
          v_new.data_ptr(), _lib.SRC_F16 if k_new.dtype == torch.float16 else _lib.SRC_F32,
          seq_len.data_ptr(), n_seq, n_pos, max_seq_len, out.data_ptr(), _ptr(sel), _ptr(n_sel), ws.ptr(),
@@ -477,9 +502,9 @@ def sparse_attn_decode_noalloc(cache: KvCache, q: torch.Tensor, k_new: torch.Ten
     if (sel is None) != (n_sel is None):
         raise ValueError("pass both sel and n_sel or neither")
     if sel is not None:                            # the kernels write max_selected entries a (sequence, KV head)
-        _need(sel, "sel", torch.int32, n_seq * cfg.n_head_kv * cfg.max_selected(max_seq_len))
+        _need(sel, "sel", torch.int32, n_seq * cfg.n_head_kv * cache.max_selected(max_seq_len))
         _need(n_sel, "n_sel", torch.int32, n_seq * cfg.n_head_kv)
-    s = cfg.shape()
+    s = cache.c_shape()
     call("qwfn_sparse_attn_decode_noalloc", C.byref(s), C.byref(cache.view()), q.data_ptr(), k_new.data_ptr(),
          v_new.data_ptr(), _lib.SRC_F16 if k_new.dtype == torch.float16 else _lib.SRC_F32,
          seq_len.data_ptr(), n_seq, max_seq_len, out.data_ptr(), _ptr(sel), _ptr(n_sel), _stream(stream))
@@ -517,7 +542,7 @@ def sparse_attn_prefill(cache: KvCache, q: torch.Tensor, seq: int, pos0: int, ws
         _need(sel, "sel", torch.int32)
         _need(n_sel, "n_sel", torch.int32, n_q * cfg.n_head_kv)
         max_sel = sel.shape[-1]
-    s = cfg.shape()
+    s = cache.c_shape()
     call("qwfn_sparse_attn_prefill", C.byref(s), C.byref(cache.view()), q.data_ptr(), _ptr(k_new), _ptr(v_new),
          src, seq, pos0, n_q, out.data_ptr(), _ptr(sel), _ptr(n_sel), max_sel, ws.ptr(), ws.nbytes,
          _stream(stream))
@@ -540,7 +565,7 @@ def decode_append_select(cache: KvCache, q: torch.Tensor, k_new: torch.Tensor, v
     _need(seq_len, "seq_len", torch.int32)
     _need(sel, "sel", torch.int32)
     _need(n_sel, "n_sel", torch.int32, n_seq * cfg.n_head_kv)
-    s = cfg.shape()
+    s = cache.c_shape()
     call("qwfn_decode_append_select", C.byref(s), C.byref(cache.view()), q.data_ptr(), k_new.data_ptr(),
          v_new.data_ptr(), _lib.SRC_F16 if k_new.dtype == torch.float16 else _lib.SRC_F32,
          seq_len.data_ptr(), n_seq, max_seq_len, sel.data_ptr(), n_sel.data_ptr(), sel.shape[-1], ws.ptr(),
@@ -620,6 +645,7 @@ class IdxCache:
     pooled: torch.Tensor
     k_norm: torch.Tensor
     _view: IdxView = field(default=None, repr=False)
+    _shape: tuple = field(default=None, repr=False, compare=False)
 
     @classmethod
     def allocate(cls, icfg: IdxConfig, kv: KvCache, k_norm: torch.Tensor) -> "IdxCache":
@@ -635,6 +661,12 @@ class IdxCache:
         k_norm = k_norm.to(device=dev, dtype=torch.float32).contiguous()
         _need(k_norm, "k_norm", torch.float32, icfg.idx_dim)
         return cls(icfg, kv, raw, pooled, k_norm)
+
+    def c_shape(self) -> IdxShape:
+        got = self._shape
+        if got is None or got[0] is not self.icfg:
+            got = self._shape = (self.icfg, self.icfg.shape())
+        return got[1]
 
     def view(self) -> IdxView:
         if self._view is None:
@@ -660,7 +692,7 @@ def idx_append_pool(ic: IdxCache, k_raw: torch.Tensor, pos: torch.Tensor,
     _need(pos, "pos", torch.int32)
     if seq_ids is not None:
         _need(seq_ids, "seq_ids", torch.int32, n_rows)
-    call("qwfn_idx_append_pool", C.byref(ic.kv.cfg.shape()), C.byref(ic.kv.view()), C.byref(ic.icfg.shape()),
+    call("qwfn_idx_append_pool", C.byref(ic.kv.c_shape()), C.byref(ic.kv.view()), C.byref(ic.c_shape()),
          C.byref(ic.view()), k_raw.data_ptr(), _lib.SRC_F16 if k_raw.dtype == torch.float16 else _lib.SRC_F32,
          _ptr(seq_ids), pos.data_ptr(), n_rows, _stream(stream))
 
@@ -668,7 +700,7 @@ def idx_append_pool(ic: IdxCache, k_raw: torch.Tensor, pos: torch.Tensor,
 def idx_pool_rebuild(ic: IdxCache, seq: int, n_whole: int, stream=None) -> None:
     """Pool the indexer keys of blocks [0, n_whole) of ``seq`` (qsa_pool_rebuild,
     src/qwfn_graph.cpp:431-448)."""
-    call("qwfn_idx_pool_rebuild", C.byref(ic.kv.cfg.shape()), C.byref(ic.kv.view()), C.byref(ic.icfg.shape()),
+    call("qwfn_idx_pool_rebuild", C.byref(ic.kv.c_shape()), C.byref(ic.kv.view()), C.byref(ic.c_shape()),
          C.byref(ic.view()), seq, n_whole, _stream(stream))
 
 
@@ -678,18 +710,18 @@ def idx_select(ic: IdxCache, q_idx: torch.Tensor, seq_len: torch.Tensor, max_seq
     sequence (src/qwfn_graph.cpp:477-495): q_idx [n_seq, n_idx_head, idx_dim]
     (normed and rotated).  Returns (sel [n_seq, n_head_kv, max_sel], n_sel
     [n_seq, n_head_kv]) with one selection repeated for every KV head."""
-    cfg, icfg = ic.kv.cfg, ic.icfg
+    cache, cfg, icfg = ic.kv, ic.kv.cfg, ic.icfg
     n_seq = seq_len.numel()
     _need(q_idx, "q_idx", torch.float32, n_seq * icfg.n_idx_head * icfg.idx_dim)
     _need(seq_len, "seq_len", torch.int32)
-    max_sel = cfg.max_selected(max_seq_len)
+    max_sel = cache.max_selected(max_seq_len)
     if sel is None:
         sel = torch.empty((n_seq, cfg.n_head_kv, max_sel), dtype=torch.int32, device=q_idx.device)
     if n_sel is None:
         n_sel = torch.empty((n_seq, cfg.n_head_kv), dtype=torch.int32, device=q_idx.device)
     _need(sel, "sel", torch.int32)
     _need(n_sel, "n_sel", torch.int32, n_seq * cfg.n_head_kv)
-    call("qwfn_idx_select", C.byref(cfg.shape()), C.byref(ic.kv.view()), C.byref(icfg.shape()), C.byref(ic.view()),
+    call("qwfn_idx_select", C.byref(ic.kv.c_shape()), C.byref(ic.kv.view()), C.byref(ic.c_shape()), C.byref(ic.view()),
          q_idx.data_ptr(), seq_len.data_ptr(), n_seq, max_seq_len, sel.data_ptr(), n_sel.data_ptr(), sel.shape[-1],
          ws.ptr(), ws.nbytes, _stream(stream))
     return sel, n_sel
@@ -717,7 +749,7 @@ def idx_sparse_attn_decode(ic: IdxCache, q: torch.Tensor, q_idx: torch.Tensor, k
     _need(v_new, "v_new", k_new.dtype, n_seq * cfg.kv_dim)
     _need(k_raw, "k_raw", k_new.dtype, n_seq * icfg.idx_dim)
     _need(seq_len, "seq_len", torch.int32)
-    max_sel = cfg.max_selected(max_seq_len)
+    max_sel = cache.max_selected(max_seq_len)
     if sel is None:
         sel = torch.empty((n_seq, cfg.n_head_kv, max_sel), dtype=torch.int32, device=q.device)
     if n_sel is None:
@@ -729,7 +761,7 @@ def idx_sparse_attn_decode(ic: IdxCache, q: torch.Tensor, q_idx: torch.Tensor, k
     if out is None:
         out = torch.empty((n_seq, cfg.n_head, cfg.head_dim), dtype=torch.float32, device=q.device)
     _need(out, "out", torch.float32, n_seq * cfg.n_head * cfg.head_dim)
-    call("qwfn_idx_sparse_attn_decode", C.byref(cfg.shape()), C.byref(cache.view()), C.byref(icfg.shape()),
+    call("qwfn_idx_sparse_attn_decode", C.byref(ic.kv.c_shape()), C.byref(cache.view()), C.byref(ic.c_shape()),
          C.byref(ic.view()), q.data_ptr(), q_idx.data_ptr(), k_new.data_ptr(), v_new.data_ptr(), k_raw.data_ptr(),
          _lib.SRC_F16 if k_new.dtype == torch.float16 else _lib.SRC_F32, seq_len.data_ptr(), n_seq, max_seq_len,
          out.data_ptr(), sel.data_ptr(), n_sel.data_ptr(), sel.shape[-1], ws.ptr(), ws.nbytes, _stream(stream))
@@ -771,7 +803,7 @@ def idx_sparse_attn_prefill(ic: IdxCache, q: torch.Tensor, q_idx: torch.Tensor, 
         _need(sel, "sel", torch.int32)
         _need(n_sel, "n_sel", torch.int32, n_q * cfg.n_head_kv)
         max_sel = sel.shape[-1]
-    call("qwfn_idx_sparse_attn_prefill", C.byref(cfg.shape()), C.byref(cache.view()), C.byref(icfg.shape()),
+    call("qwfn_idx_sparse_attn_prefill", C.byref(ic.kv.c_shape()), C.byref(cache.view()), C.byref(ic.c_shape()),
          C.byref(ic.view()), q.data_ptr(), q_idx.data_ptr(), _ptr(k_new), _ptr(v_new), _ptr(k_raw), src, seq,
          pos0, n_q, out.data_ptr(), _ptr(sel), _ptr(n_sel), max_sel, ws.ptr(), ws.nbytes, _stream(stream))
     return out
