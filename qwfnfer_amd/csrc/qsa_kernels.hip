@@ -1394,8 +1394,169 @@ k_kv_rows(Geo g, qwfn_kv_view v, int32_t seq, int32_t pos0, int32_t n, uint8_t *
     }
 }
 
+// Many tokens of rows that 16-byte loads can take: a workgroup a 64-token tile and
+// side (K, V).  The tile's rows are one contiguous range, moved in 16-byte pieces
+// between the rows and LDS, and its page bytes in 16-byte chunks between LDS and the
+// page; the 2-byte alignment of a q8_0 or q4_0 row's quants inside and the transpose
+// of dim-major V stay in LDS.  Bound by HBM: K and V of 65,537 tokens, q8_0, are
+// 35.7 MB read and as much written in 14.7 us either way (4.9 TB/s); a block a thread,
+// whose 34-byte strides and single bytes of V fill no line at once, 33.5.
+// LDS rows are padded by a dword: consecutive rows start on consecutive banks.
+// In a tile that the call covers in part only its own tokens' bytes are written, one
+// by one where dim-major V packs 16 tokens in a chunk.
+using u16_alias = uint16_t __attribute__((may_alias));
+constexpr size_t kKvRowLds = 65536;                // the widest tile that takes this path
+
+// byte of 16-byte chunk c of KV head gh inside a row
+__device__ __forceinline__ int row_chunk_off(const Geo &g, int gh, int c) {
+    const int nb = g.hd / 32;
+    if (g.kt == QWFN_KV_F16) return (gh * g.chunks + c) * 16;
+    if (g.kt == QWFN_KV_Q4_0) return (gh * nb + c) * 18 + 2;
+    return (gh * nb + c / 2) * 34 + 2 + (c & 1) * 16;
+}
+
+// 4x4 bytes: out[k] = byte k of r[0..3]
+__device__ __forceinline__ void transpose4(const uint32_t r[4], uint32_t out[4]) {
+    const uint32_t a = __builtin_amdgcn_perm(r[1], r[0], 0x05010400u), b = __builtin_amdgcn_perm(r[3], r[2], 0x05010400u);
+    const uint32_t c = __builtin_amdgcn_perm(r[1], r[0], 0x07030602u), d = __builtin_amdgcn_perm(r[3], r[2], 0x07030602u);
+    out[0] = __builtin_amdgcn_perm(b, a, 0x05040100u);
+    out[1] = __builtin_amdgcn_perm(b, a, 0x07060302u);
+    out[2] = __builtin_amdgcn_perm(d, c, 0x05040100u);
+    out[3] = __builtin_amdgcn_perm(d, c, 0x07060302u);
+}
+
+template <bool EXPORT>
+__global__ void __launch_bounds__(256)
+k_kv_tiles(Geo g, qwfn_kv_view v, int32_t seq, int32_t pos0, int32_t n, int32_t row_bytes, uint8_t *k_rows,
+           uint8_t *v_rows) {
+    extern __shared__ uint32_t kv_lds[];
+    const bool is_v = blockIdx.y != 0;
+    uint8_t *rows = is_v ? v_rows : k_rows;
+    if (!rows) return;
+    const int tile = pos0 / 64 + blockIdx.x, tid = threadIdx.x;
+    const int lo = max(pos0 - tile * 64, 0), hi = min(n - (tile * 64 - pos0), 64);   // the tile's tokens [lo, hi)
+    const int32_t pp = phys_page(g, v.page_table, seq, tile * 64);
+    if (pp < 0) { if (tid == 0) set_status(v.status, QWFN_STATUS_PAGE_RANGE); return; }
+    uint8_t *page = (uint8_t *)(is_v ? v.v_pages : v.k_pages) + (int64_t)pp * g.page_bytes;
+    const int row0 = tile * 64 % g.pt;             // the tile's first row in its page
+    rows += (int64_t)(tile * 64 + lo - pos0) * row_bytes;
+    const int pieces = row_bytes / 16, stride = row_bytes / 4 + 1;
+    const int nb = g.hd / 32, nscale = g.kt == QWFN_KV_F16 ? 0 : 64 * nb * g.Hkv;
+    const int blk = g.kt == QWFN_KV_Q4_0 ? 18 : 34;
+    u16_alias *h16 = reinterpret_cast<u16_alias *>(kv_lds);
+    const bool dimv = is_v && g.vdim;
+
+    const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
+    const int r_step = 256 / pieces, p_step = 256 % pieces;       // a thread's next piece: no division
+
+    if (!EXPORT) {
+        for (int i = tid, r = lo + tid / pieces, p = tid % pieces; i < (hi - lo) * pieces; i += 256) {
+            const uint4 x = reinterpret_cast<const uint4 *>(rows)[i];
+            uint32_t *d = kv_lds + r * stride + p * 4;
+            d[0] = x.x; d[1] = x.y; d[2] = x.z; d[3] = x.w;
+            r += r_step, p += p_step;
+            if (p >= pieces) p -= pieces, ++r;
+        }
+        __syncthreads();
+    }
+    if (!dimv) {                                   // a chunk of 64 tokens a wave
+        const int r = tid % 64;
+        for (int x = wave; x < g.chunks * g.Hkv; x += 4) {
+            const int gh = x / g.chunks, c = x - gh * g.chunks;
+            if (r < lo || r >= hi) continue;
+            uint4 *cp = reinterpret_cast<uint4 *>(page + chunk_off(g, gh, row0 + r, c));
+            u16_alias *l = h16 + (2 * r * stride + row_chunk_off(g, gh, c) / 2);
+            uint32_t w[4];
+            if (EXPORT) {
+                const uint4 x = *cp;
+                w[0] = x.x; w[1] = x.y; w[2] = x.z; w[3] = x.w;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) { l[2 * k] = (uint16_t)w[k]; l[2 * k + 1] = (uint16_t)(w[k] >> 16); }
+            } else {
+#pragma unroll
+                for (int k = 0; k < 4; ++k) w[k] = (uint32_t)l[2 * k] | ((uint32_t)l[2 * k + 1] << 16);
+                *cp = make_uint4(w[0], w[1], w[2], w[3]);
+            }
+        }
+    } else {                                       // four dims of sixteen tokens a thread
+        for (int i = tid; i < g.hd * g.Hkv; i += 256) {
+            const int tg = i % 4 * 16, d = i / 4 * 4 % g.hd, gh = i / 4 * 4 / g.hd;
+            uint8_t *p = page + vquant_off(g, gh, row0 + tg, d);
+            u16_alias *l = h16 + (2 * tg * stride + ((gh * nb + d / 32) * 34 + 2 + d % 32) / 2);
+            const bool whole = tg >= lo && tg + 16 <= hi;
+            uint32_t w[4][4];                      // [dim][four tokens]
+            if (EXPORT) {
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    const uint4 x = *reinterpret_cast<const uint4 *>(p + 64 * k);
+                    w[k][0] = x.x; w[k][1] = x.y; w[k][2] = x.z; w[k][3] = x.w;
+                }
+            }
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                uint32_t a[4], b[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    const u16_alias *e = l + 2 * (4 * q + k) * stride;
+                    a[k] = EXPORT ? w[k][q] : (uint32_t)e[0] | ((uint32_t)e[1] << 16);
+                }
+                transpose4(a, b);
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    u16_alias *e = l + 2 * (4 * q + k) * stride;
+                    if (EXPORT) { e[0] = (uint16_t)b[k]; e[1] = (uint16_t)(b[k] >> 16); }
+                    else w[k][q] = b[k];
+                }
+            }
+            if (EXPORT) continue;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                if (whole) {
+                    *reinterpret_cast<uint4 *>(p + 64 * k) = make_uint4(w[k][0], w[k][1], w[k][2], w[k][3]);
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 16; ++e)
+                        if (tg + e >= lo && tg + e < hi) p[64 * k + e] = (uint8_t)(w[k][e / 4] >> (e % 4 * 8));
+                }
+            }
+        }
+    }
+    for (int i = tid; i < nscale; i += 256) {      // a head's scales of a tile are contiguous
+        const int y = i / nb, j = i - y * nb, r = y % 64, gh = y / 64;
+        if (r < lo || r >= hi) continue;
+        uint16_t *sp = reinterpret_cast<uint16_t *>(page + scale_off(g, gh, row0 + r, j));
+        u16_alias *l = h16 + (2 * r * stride + (gh * nb + j) * blk / 2);
+        if (EXPORT) *l = *sp;
+        else *sp = *l;
+    }
+    if (EXPORT) {
+        __syncthreads();
+        for (int i = tid, r = lo + tid / pieces, p = tid % pieces; i < (hi - lo) * pieces; i += 256) {
+            const uint32_t *d = kv_lds + r * stride + p * 4;
+            reinterpret_cast<uint4 *>(rows)[i] = make_uint4(d[0], d[1], d[2], d[3]);
+            r += r_step, p += p_step;
+            if (p >= pieces) p -= pieces, ++r;
+        }
+    }
+}
+
+// Whole tiles where the rows are 16-byte aligned, from 64 tokens; below that, for rows
+// at other addresses and for rows from 1,024 bytes (their tile is past the 64 KB of LDS
+// a launch may ask for) the kernel of one block a thread.  Import, pooling and export
+// together, two KV heads of 128: 163,840 tokens q8_0 184 -> 81 us, fp16 218 -> 154,
+// q4_0 51 both (its 144-byte rows were read in place already); up to 8,192 tokens the
+// three calls' 22 us on the host hide either kernel.
 hipError_t launch_kv_rows(const Geo &g, const qwfn_kv_view &v, bool to_rows, int32_t seq, int32_t pos0,
                           int32_t n, void *k_rows, void *v_rows, hipStream_t st) {
+    const int rb = g.kt == QWFN_KV_F16 ? g.Hkv * g.hd * 2 : g.Hkv * (g.hd / 32) * (g.kt == QWFN_KV_Q4_0 ? 18 : 34);
+    const size_t lds = 64u * (rb + 4);
+    if (n >= 64 && rb % 16 == 0 && lds <= kKvRowLds && (((uintptr_t)k_rows | (uintptr_t)v_rows) & 15) == 0) {
+        const int64_t tiles = ((int64_t)pos0 + n + 63) / 64 - pos0 / 64;
+        const dim3 grid((unsigned)tiles, v_rows ? 2u : 1u);
+        hipLaunchKernelGGL(to_rows ? k_kv_tiles<true> : k_kv_tiles<false>, grid, dim3(256), lds, st, g, v, seq,
+                           pos0, n, rb, (uint8_t *)k_rows, (uint8_t *)v_rows);
+        return hipGetLastError();
+    }
     const int64_t threads = (int64_t)n * g.Hkv * (g.hd / 32);
     const dim3 grid((unsigned)((threads + 255) / 256));
     if (to_rows)

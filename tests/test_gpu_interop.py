@@ -7,6 +7,8 @@ quantization of the appended values in that order, byte for byte; imported
 rows must leave the bytes an append would; a snapshot must reproduce the
 selections and attention of the cache it came from, bit for bit.
 """
+import dataclasses
+
 import numpy as np
 import pytest
 import torch
@@ -97,6 +99,43 @@ def test_any_bytes_round_trip():
         k2, v2 = qsa.export_rows_q8_0(dev, 0, pos0, n)
         torch.cuda.synchronize()
         assert torch.equal(k2, kr) and torch.equal(v2, vr)
+
+
+@pytest.mark.parametrize("kv", [_lib.KV_Q8_0, _lib.KV_Q4_0, _lib.KV_F16])
+@pytest.mark.parametrize("cfg", [BASELINE, TINY, G12, dataclasses.replace(G12, block_tokens=64, top_k_blocks=8)])
+def test_row_addresses_do_not_change_the_bytes(cfg, kv):
+    """Rows at 16-byte addresses go a tile at a time, rows at other 2-byte addresses a
+    block at a time: both leave the same page bytes, touch no other token's, and export
+    what was imported.  Whole tiles, one tile short of and past whole, ragged at both ends."""
+    c = dataclasses.replace(cfg_of(cfg), kv_type=kv)
+    rb, pps = c.row_bytes(), 4
+    gen = torch.Generator().manual_seed(77)
+    bytes_of = lambda *shape: torch.randint(0, 256, shape, dtype=torch.uint8, generator=gen).cuda()
+    caches = []
+    for _ in range(2):
+        pt = torch.tensor([[3, 0, 4, 1]], dtype=torch.int32)
+        caches.append(qsa.KvCache.allocate(c, 1, pps, page_table=pt, n_phys_pages=5))
+    tokens = pps * c.page_tokens
+    for pos0, n in ((0, 64), (0, tokens), (64, 65), (37, 64), (63, 130 if tokens > 200 else 65), (1, tokens - 2),
+                    (tokens - 64, 64), (5, 63)):
+        base = bytes_of(2, caches[0].k_pages.numel())
+        src = bytes_of(2, n * rb + 16)
+        for cache, off in zip(caches, (0, 2)):
+            cache.k_pages.view(torch.uint8).view(-1).copy_(base[0])
+            cache.v_pages.view(torch.uint8).view(-1).copy_(base[1])
+            rows = torch.empty((2, n * rb + 32 - n * rb % 16), dtype=torch.uint8, device="cuda")
+            kr, vr = (rows[i, off:off + n * rb].view(n, rb) for i in range(2))
+            assert kr.data_ptr() % 16 == off and vr.data_ptr() % 16 == off
+            kr.copy_(src[0, :n * rb].view(n, rb))
+            vr.copy_(src[1, :n * rb].view(n, rb))
+            qsa.import_rows_q8_0(cache, 0, pos0, kr, vr)
+            ke, ve = qsa.export_rows_q8_0(cache, 0, pos0, n)
+            assert torch.equal(ke, kr) and torch.equal(ve, vr), (pos0, n, off)
+            only, none = qsa.export_rows_q8_0(cache, 0, pos0, n, k=False)
+            assert only is None and torch.equal(none, vr)
+        assert torch.equal(caches[0].k_pages, caches[1].k_pages), (pos0, n)
+        assert torch.equal(caches[0].v_pages, caches[1].v_pages), (pos0, n)
+    assert all(qsa.read_status(cache) == 0 for cache in caches)
 
 
 def test_bad_page_entries_set_the_status_bit():
