@@ -798,7 +798,7 @@ static hipError_t launch_indexer_t(const Geo &g, const qwfn_kv_view &v, const fl
 // count recomputed from the length and the selection as the attention counts
 // it).  Thread (r, d), r = tid / HD (uniform in a wave), sums dimension d over
 // the parts congruent to r mod R.  The length, the count, the (max, sum)
-// pairs of parts lane and lane + 64, and the thread's first U part rows all go
+// pairs of parts lane + 64 k, and the thread's first U part rows all go
 // out in the first round trip (rows clamped to the most parts the attention
 // can write, inside the pair's n_tiles rows).  Every wave reduces the maxima
 // and weighted sums itself and takes a part's weight from the lane holding it
@@ -806,14 +806,17 @@ static hipError_t launch_indexer_t(const Geo &g, const qwfn_kv_view &v, const fl
 // gives zeros (and, for a length, the status bit).
 // grid (G, Hkv, n_seq or n_q), R * head_dim threads
 template <int HD> constexpr int merge_r() { return HD > 128 ? 2 : 4; }
-constexpr int kMergeRound = 24;                   // part rows a thread loads in one round
-template <int G, int HD>
+// U, the part rows a thread loads in one round: kMergeRound, or kMergeWide where
+// the call can leave more parts than that round takes (the dense layer's, one a
+// tile): the next rounds' rows and weights wait on the first's.
+constexpr int kMergeRound = 24, kMergeWide = 64;
+template <int G, int HD, int U>
 __global__ void __launch_bounds__(merge_r<HD>() * HD)
 k_merge(Geo g, qwfn_kv_view v, const int32_t *seq_len, int32_t max_seq_len, const int32_t *nsel,
         int32_t max_sel, int32_t dense, float *__restrict__ out, Ws ws, int32_t tg) {
 #pragma clang fp contract(off)
-    constexpr int R = merge_r<HD>(), U = kMergeRound, PR = R * U;   // parts a round
-    static_assert(PR <= 128 && HD % 64 == 0, "round weights in two lanes' registers; whole waves");
+    constexpr int R = merge_r<HD>(), PR = R * U, W = (PR + 63) / 64;   // parts a round; W registers hold their weights
+    static_assert(HD % 64 == 0 && 64 % R == 0, "whole waves; the R parts of a step in one register");
     __shared__ float red[R][HD];
     const int h = blockIdx.x, gh = blockIdx.y, s = blockIdx.z;
     const int tid = threadIdx.x, d = tid % HD, r = tid / HD, lane = tid & 63;
@@ -825,9 +828,9 @@ k_merge(Geo g, qwfn_kv_view v, const int32_t *seq_len, int32_t max_seq_len, cons
     const float *pml = ws.part_ml + row * 2;
     const float *po = ws.part_o + row * HD + d;
     const int last = (ws.n_tiles + tg - 1) / tg - 1;
-    float2 ml[2];
+    float2 ml[W];
 #pragma unroll
-    for (int k = 0; k < 2; ++k)
+    for (int k = 0; k < W; ++k)
         ml[k] = *reinterpret_cast<const float2 *>(pml + (int64_t)min(lane + 64 * k, last) * 2 * G);
     float x[U];
 #pragma unroll
@@ -848,19 +851,19 @@ k_merge(Geo g, qwfn_kv_view v, const int32_t *seq_len, int32_t max_seq_len, cons
     auto m_of = [&](int i) { return pml[(int64_t)i * 2 * G]; };
     float mx = -INFINITY;
 #pragma unroll
-    for (int k = 0; k < 2; ++k) mx = lane + 64 * k < parts ? fmaxf(mx, ml[k].x) : mx;
-    for (int i = lane + 128; i < parts; i += 64) mx = fmaxf(mx, m_of(i));
+    for (int k = 0; k < W; ++k) mx = lane + 64 * k < parts ? fmaxf(mx, ml[k].x) : mx;
+    for (int i = lane + 64 * W; i < parts; i += 64) mx = fmaxf(mx, m_of(i));
     const float M = wave_max(mx);
     auto weight = [&](float m) { return m == -INFINITY ? 0.0f : exp2f(m - M); };
-    float wk[2];                                   // weights of parts lane, lane + 64 (0 past the parts)
+    float wk[W];                                   // weights of parts lane + 64 k (0 past the parts)
     float ls = 0.0f;
 #pragma unroll
-    for (int k = 0; k < 2; ++k) {
+    for (int k = 0; k < W; ++k) {
         const bool in = lane + 64 * k < parts;
         wk[k] = in ? weight(ml[k].x) : 0.0f;
         ls += wk[k] * (in ? ml[k].y : 0.0f);
     }
-    for (int i = lane + 128; i < parts; i += 64) ls += weight(m_of(i)) * pml[(int64_t)i * 2 * G + 1];
+    for (int i = lane + 64 * W; i < parts; i += 64) ls += weight(m_of(i)) * pml[(int64_t)i * 2 * G + 1];
     const float Ls = wave_sum(ls);
     // straight-line over the round: a part past the count has weight 0 and
     // its row, not written by this call, is replaced by 0
@@ -868,9 +871,8 @@ k_merge(Geo g, qwfn_kv_view v, const int32_t *seq_len, int32_t max_seq_len, cons
 #pragma unroll
     for (int u = 0; u < U; ++u) {
         const int p = r + R * u;                   // wave-uniform
-        const int w0 = __builtin_amdgcn_readlane(__builtin_bit_cast(int, wk[0]), p & 63);
-        const int w1 = __builtin_amdgcn_readlane(__builtin_bit_cast(int, wk[1]), p & 63);
-        const float wp = __builtin_bit_cast(float, p < 64 ? w0 : w1);
+        const int w = __builtin_amdgcn_readlane(__builtin_bit_cast(int, wk[R * u / 64]), p & 63);
+        const float wp = __builtin_bit_cast(float, w);
         acc += wp * (p < parts ? x[u] : 0.0f);
     }
     for (int i0 = PR; i0 < parts; i0 += PR) {     // more parts than one round
@@ -894,13 +896,24 @@ k_merge(Geo g, qwfn_kv_view v, const int32_t *seq_len, int32_t max_seq_len, cons
     }
 }
 
+// The wide round past merge_r * kMergeRound parts while the grid is at most one
+// workgroup a CU, all that its 206 registers leave room for.  The sums and their order
+// are the same in either.  Dense decode over fp16, one token: 16,001 tokens (251 parts)
+// 22.0 us a call with rounds of 24, 19.5 wide; 65,536 tokens 42.3, 38.3; 7,000 tokens
+// (110 parts) the same; 32 sequences to 16,001, 512 workgroups: 67.6, 71.6.
 template <int G, int HD>
 static void launch_merge_t(const Geo &g, const qwfn_kv_view &v, const int32_t *seq_len, int32_t n_seq,
-                           int32_t max_seq_len, const int32_t *sel, const int32_t *nsel, int32_t max_sel,
-                           float *out, const Ws &ws, int32_t tg, hipStream_t st) {
-    QWFN_LAUNCH(kTimedMerge, (k_merge<G, HD>), dim3((unsigned)G, (unsigned)g.Hkv, (unsigned)n_seq),
-                dim3(merge_r<HD>() * HD), st, g, v, seq_len, max_seq_len, nsel, max_sel, (int32_t)(sel == nullptr), out,
-                ws, tg);
+                           int32_t max_seq_len, const int32_t *nsel, int32_t max_sel, bool dense, float *out,
+                           const Ws &ws, int32_t tg, hipStream_t st) {
+    const dim3 grid((unsigned)G, (unsigned)g.Hkv, (unsigned)n_seq), blk(merge_r<HD>() * HD);
+    const bool wide = (ws.n_tiles + tg - 1) / tg > merge_r<HD>() * kMergeRound &&
+                      (int64_t)G * g.Hkv * n_seq <= device_cus();
+    if (wide)
+        QWFN_LAUNCH(kTimedMerge, (k_merge<G, HD, kMergeWide>), grid, blk, st, g, v, seq_len, max_seq_len, nsel,
+                    max_sel, (int32_t)dense, out, ws, tg);
+    else
+        QWFN_LAUNCH(kTimedMerge, (k_merge<G, HD, kMergeRound>), grid, blk, st, g, v, seq_len, max_seq_len, nsel,
+                    max_sel, (int32_t)dense, out, ws, tg);
 }
 
 #define QWFN_FOR_EACH_MERGE(X) X(128, 8) X(128, 4) X(128, 2) X(64, 8) X(256, 12) X(256, 8)
@@ -909,9 +922,7 @@ hipError_t launch_merge(const Geo &g, const qwfn_kv_view &v, const int32_t *seq_
                         const Ws &ws, int32_t tg, hipStream_t st) {
 #define X(HD_, G_)                                                                                            \
     if (g.hd == HD_ && g.G == G_) {                                                                           \
-        QWFN_LAUNCH(kTimedMerge, (k_merge<G_, HD_>), dim3((unsigned)G_, (unsigned)g.Hkv, (unsigned)n_seq),    \
-                    dim3(merge_r<HD_>() * HD_), st, g, v, seq_len, max_seq_len, nsel, max_sel, (int32_t)dense, out, ws, \
-                    tg);                                                                                      \
+        launch_merge_t<G_, HD_>(g, v, seq_len, n_seq, max_seq_len, nsel, max_sel, dense, out, ws, tg, st);    \
         return hipGetLastError();                                                                             \
     }
     QWFN_FOR_EACH_MERGE(X)
@@ -1268,7 +1279,7 @@ static void launch_attn_t(const Geo &g, const qwfn_kv_view &v, const float *q,
     else
         QWFN_LAUNCH(kTimedAttention, (k_attn<HD, G, TG, QWFN_KV_Q8_0>), grid, blk, st, g, v, q, seq_len, max_seq_len,
                     sel, nsel, max_sel, out, ws, n_parts);
-    launch_merge_t<G, HD>(g, v, seq_len, n_seq, max_seq_len, sel, nsel, max_sel, out, ws, TG, st);
+    launch_merge_t<G, HD>(g, v, seq_len, n_seq, max_seq_len, nsel, max_sel, sel == nullptr, out, ws, TG, st);
 }
 
 // The general attention selecting for itself (SEL): sel / nsel are outputs.
@@ -1289,7 +1300,7 @@ static void launch_attn_sel_t(const Geo &g, const qwfn_kv_view &v, const float *
     else
         QWFN_LAUNCH(kTimedAttention, (k_attn<HD, G, TG, QWFN_KV_Q8_0, true>), grid, blk, st, g, v, q, seq_len,
                     max_seq_len, sel, nsel, max_sel, out, ws, n_parts);
-    launch_merge_t<G, HD>(g, v, seq_len, n_seq, max_seq_len, sel, nsel, max_sel, out, ws, TG, st);
+    launch_merge_t<G, HD>(g, v, seq_len, n_seq, max_seq_len, nsel, max_sel, sel == nullptr, out, ws, TG, st);
 }
 
 // ---------------------------------------------------------------------------

@@ -193,3 +193,26 @@ def test_batched_attention_wide_v_scales():
     sel = np.broadcast_to(np.arange(nb, dtype=np.int32), (1, cfg.n_head_kv, nb)).copy()
     ref = host.attention_f64(q, np.array([L], np.int32), sel, np.full((1, cfg.n_head_kv), nb, np.int32))
     assert_close_attn(np_of(out), ref)
+
+
+# Dense decode leaves a part a tile; the merge takes up to 24 or 64 of them a thread
+# at once, four threads a dimension (two past 128 dimensions): parts on both sides of
+# both counts, and beside each longest sequence one token and a middle length, whose
+# parts end long before.
+@pytest.mark.parametrize("cfg, parts", [
+    (Cfg(top_k_blocks=0), 96), (Cfg(top_k_blocks=0), 97), (Cfg(top_k_blocks=0), 256), (Cfg(top_k_blocks=0), 257),
+    (Cfg(top_k_blocks=0, head_dim=256), 49), (Cfg(top_k_blocks=0, head_dim=256), 129),
+    (Cfg(top_k_blocks=0, kv_type=2), 130),
+])
+def test_dense_merge_of_many_parts(cfg, parts):
+    lengths = [64 * parts, 1, 64 * (parts - 1) // 2 + 7]
+    rng = np.random.default_rng(parts)
+    dev, host = make_pair(cfg, 3, lengths[0] // cfg.page_tokens + 1, seed=9)
+    fill(dev, host, rng, lengths, pool=False)
+    q = rng.standard_normal((3, cfg.n_head, cfg.head_dim), dtype=np.float32)
+    L = np.array(lengths, np.int32)
+    ws = qsa.Workspace(cfg_of(cfg), 3, int(L.max()))
+    out = qsa.sparse_decode_attn(dev, torch.from_numpy(q).cuda(), torch.from_numpy(L).cuda(), int(L.max()), ws)
+    torch.cuda.synchronize()
+    assert qsa.read_status(dev) == 0
+    assert_close_attn(np_of(out), host.attention_f64(q, L), f"dense, {parts} parts")
