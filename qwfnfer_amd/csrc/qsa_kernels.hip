@@ -2366,7 +2366,7 @@ k_pf_refine(Geo g, qwfn_kv_view v, const float *__restrict__ q, float *scores, i
 // (a single KV head, or a selection shared by every KV head through one
 // scoring head group: the checkpoint indexer's 4-token blocks): one
 // 1024-thread workgroup per query, thread t holding the 4-block groups
-// base + 4 (t + 1024 j), j < kRbKpt / 4 (base = e_lo rounded down to a
+// base + 4 (t + 1024 j), j < KPT / 4 (base = e_lo rounded down to a
 // multiple of 4: coalesced 16-byte loads; every 64-lane wave row then covers
 // 256 consecutive blocks, in block order by (j, wave, lane)), up to kRbMax
 // candidates; the LDS of k_select_big, whose
@@ -2387,14 +2387,19 @@ struct RefineBigShared {
 // grid (1, n_q), kRbThreads: query s's selection (g.Hkv == 1; with a shared
 // selection every KV head's row) from k_pf_approx's scores, by the bound and
 // candidate argument of k_pf_refine.
-template <int HD, int G>
+// KPT, the blocks a thread holds (at most kRbKpt): every one is loaded, bounded and
+// binned whether the row reaches it or not, so the launch takes the fewest that hold
+// the longest query's row: the checkpoint's 1,900 queries at 40,003 tokens (10,476
+// blocks) 426 us with 40 a thread, 303 with 12; whole prefill calls of 1,500 queries
+// at 47,000 tokens 944 us, 855, at 90,000 (24 a thread) 1,097, 1,009.
+template <int HD, int G, int KPT>
 __global__ void __launch_bounds__(kRbThreads)
 k_pf_refine_big(Geo g, qwfn_kv_view v, const float *__restrict__ q, float *scores, int32_t nb_cap,
                 const float *__restrict__ pnorm, int32_t *sel, int32_t *nsel, int32_t max_sel) {
 #pragma clang fp contract(off)
-    constexpr int NT = kRbThreads, QS = HD + 4, KPT = kRbKpt, NW = NT / 64, NCH = HD / 16;
+    constexpr int NT = kRbThreads, QS = HD + 4, NW = NT / 64, NCH = HD / 16;
     constexpr int NJ = KPT / 4, NG = NJ * NW;          // 4-block groups a thread; (j, wave) rows
-    static_assert(pf_approx_fits<HD, G>() && G * HD / 4 <= NT && G <= NW && KPT % 4 == 0 && NG <= NT, "shapes");
+    static_assert(pf_approx_fits<HD, G>() && G * HD / 4 <= NT && G <= NW && KPT % 4 == 0 && KPT <= kRbKpt && NG <= NT, "shapes");
     __shared__ RefineBigShared<HD, G> sh;
     const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int s = blockIdx.y;
@@ -2634,8 +2639,14 @@ static void launch_pf_index_t(const Geo &g, const qwfn_kv_view &v, const float *
             n_blk - g.sink <= kRbBlocks) {
             launch_pf_approx<HD, G>(g, pa_grid(n_q, n_blk - g.sink, 1, kPaSplitBig), v, q, n_q, n_blk, ws.scores,
                                     ws.nb_cap, ws.pnorm, st);
-            hipLaunchKernelGGL((k_pf_refine_big<HD, G>), dim3(1u, (unsigned)n_q), dim3(kRbThreads), 0, st, g, v, q,
-                               ws.scores, ws.nb_cap, ws.pnorm, sel, nsel, max_sel);
+            const int span = n_blk - (g.sink & ~3);    // from the first group's first block
+#define QWFN_REFINE_BIG(KPT_)                                                                                  \
+    hipLaunchKernelGGL((k_pf_refine_big<HD, G, KPT_>), dim3(1u, (unsigned)n_q), dim3(kRbThreads), 0, st, g, v, q, \
+                       ws.scores, ws.nb_cap, ws.pnorm, sel, nsel, max_sel)
+            if (span <= 12 * kRbThreads) QWFN_REFINE_BIG(12);
+            else if (span <= 24 * kRbThreads) QWFN_REFINE_BIG(24);
+            else QWFN_REFINE_BIG(kRbKpt);
+#undef QWFN_REFINE_BIG
             return;
         }
         // per-KV-head selections (or one KV head's row shared), up to kRefineBlocks eligible blocks

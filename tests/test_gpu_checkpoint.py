@@ -517,14 +517,14 @@ def test_per_head_selection_long_context():
     assert qsa.read_status(dev) == 0
 
 
-def _long_prefill(seed, raw_keys=None):
-    """A 37-query chunk appended at 36,001 (over 9,000 eligible 4-token blocks
-    a query): selections bit for bit against the oracle's on the pooled keys
+def _long_prefill(seed, raw_keys=None, pre=36001):
+    """A 37-query chunk appended at `pre` (36,001: over 9,000 eligible 4-token
+    blocks a query): selections bit for bit against the oracle's on the pooled keys
     the device built, every ninth query's attention within tolerance.
     raw_keys(rng, n, t0) gives the indexer's raw keys of tokens t0 .. t0+n-1."""
     cfg = CKPT
     rng = np.random.default_rng(seed)
-    pre, n_q = 36001, 37
+    n_q = 37
     end = pre + n_q
     pps = end // cfg.page_tokens + 1
     dev, host, ic, w = _pair(cfg, 1, pps, seed=seed + 1)
@@ -567,6 +567,13 @@ def test_checkpoint_prefill_long_context():
     """Prefill queries at positions past 32,768 (over 8192 eligible blocks
     each): the bounded scoring and the 1024-thread refinement of one shared row."""
     _long_prefill(870)
+
+
+@pytest.mark.parametrize("end", [49155, 49156, 98311])
+def test_checkpoint_prefill_row_lengths(end):
+    """Rows on both sides of the blocks a refinement's thread holds: 12,288 blocks
+    fill 12 a thread, one more takes 24, and past 24,576 it is 40."""
+    _long_prefill(875, pre=end - 37)
 
 
 def _class_keys(classes):
