@@ -381,9 +381,9 @@ int qwfn_sparse_attn_decode_chain(const qwfn_qsa_shape *shape, const qwfn_kv_vie
  * cannot allocate device memory (code under hipGraph capture that may not
  * call hipMalloc, tight serving loops, harnesses that forbid allocation).  No
  * counterpart in the reference.  The workspace is a file-scope device array
- * of the library, 8 MiB per device, held until the process ends: calls whose
- * qwfn_qsa_workspace_bytes(shape, n_seq, max_seq_len) exceeds it return
- * QWFN_ERANGE (8 MiB holds eight sequences of the BASELINE shape up to 1M
+ * of the library, 8 MiB per device, held until the process ends: calls that
+ * need more for their one position (qwfn_qsa_workspace_bytes without the rows
+ * it adds for chained positions) return QWFN_ERANGE (8 MiB holds eight sequences of the BASELINE shape up to 1M
  * tokens).  The first call on a device enqueues one fill kernel on `stream`
  * that clears the array, unless `stream` is capturing (the array is zero when
  * the library loads, and a captured fill would rerun on every replay).  Every
