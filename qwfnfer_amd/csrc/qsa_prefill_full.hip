@@ -44,6 +44,9 @@ struct FullCfg {
     static constexpr int VPLANE = 8 * VGRP;
     static constexpr int KCH = LY == kPlQ4 ? HD / 32 : LY == kPlF16 ? HD / 8 : HD / 16;   // 16-byte chunks of a row
     static constexpr int KPIECES = KCH * 64 / 256;         // chunks a thread converts a tile
+    // kPlQ8: the 32-dim V blocks that a wave's HD / 4 dims lie in (at HD 64 two waves
+    // share a block), and the floats of its own strip of their scales, 64 cells each.
+    static constexpr int NBW = HD > 128 ? HD / 128 : 1, VSTRIP = 64 * NBW;
     static_assert(G <= COLS && KCH * 64 % 256 == 0, "whole pieces");
 };
 
@@ -61,7 +64,7 @@ struct FullK {
 template <int HD, int G, int LY>
 struct FullV {
     using C = FullCfg<HD, G, LY>;
-    float d[LY == kPlQ8 ? HD * 2 : 4];   // kPlQ8: the tile's V scales times 2^kv, 64 cells a block
+    float d[LY == kPlQ8 ? 4 * C::VSTRIP : 4];   // kPlQ8: a strip a wave of the tile's V scales times 2^kv
     // (two groups' tiles also hold a group's O at the end)
     static constexpr int BYTES = C::VP * C::VPLANE, XCH = C::GR == 2 ? 4 * C::NCT * C::ND * 1024 / 2 : 0;
     __attribute__((aligned(16))) uint8_t v[BYTES > XCH ? BYTES : XCH];
@@ -327,9 +330,11 @@ k_pf_full(Geo g, qwfn_kv_view v, const float *__restrict__ q, int32_t n_q, const
         *reinterpret_cast<uint2 *>(vdst8 + C::VPLANE + lgx * C::VGRP + d * 16) = make_uint2(x[2], x[3]);
     };
     auto conv_v8 = [&](auto put) {
-        constexpr int NP = HD / 64, NBW = NP > 2 ? NP / 2 : 1;   // dims a thread, blocks a wave
+        constexpr int NP = HD / 64, NBW = C::NBW;    // dims a thread, blocks a wave
+        static_assert(LY != kPlQ8 || (4 * C::VSTRIP <= (int)(sizeof TV.d / sizeof TV.d[0]) && 32 * NBW >= HD / 4),
+                      "four waves' strips of scales lie in the array, and hold their dims' blocks");
         const uint16_t *sc = reinterpret_cast<const uint16_t *>(&TR.v[C::KCH * 64]);
-        float *strip = TV.d + w * NBW * 64;          // the wave's own
+        float *strip = TV.d + w * C::VSTRIP;         // the wave's own
 #pragma unroll
         for (int b = 0; b < NBW; ++b) strip[64 * b + l] = h2f(sc[l * NJ + HD / 4 * w / 32 + b]) * v_up;
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");   // (a wave's LDS operations are in order)

@@ -42,6 +42,25 @@ def test_prefill_every_block(cfg, pre, n_q):
     _prefill_case(cfg, pre, n_q, seed=800 + n_q, dtype=np.float16 if n_q % 2 else np.float32)
 
 
+def _uneven_rows(rng, n, cfg):
+    """kv_rows with keys that grow along the rows (a tile's largest logit passes the
+    earlier ones for some queries and not for others) and another V scale every tile."""
+    k, v = kv_rows(rng, n, cfg)
+    k *= np.linspace(0.2, 2.0, n, dtype=np.float32)[:, None, None]
+    v *= np.exp(rng.uniform(np.log(0.1), np.log(10.0), (n // 64 + 1, 1, 1))).astype(np.float32).repeat(64, 0)[:n]
+    return k, v
+
+
+# 64-dim heads, where two waves of a tile's conversion read the scales of one 32-dim
+# block: from 512 queries (two KV heads), whole and partial query blocks and tiles.
+@pytest.mark.parametrize("pre, n_q", [(0, 512), (3, 577), (61, 1030), (640, 513)])
+def test_prefill_every_block_narrow_heads(pre, n_q):
+    print(f"narrow heads: {n_q} queries after {pre}", flush=True)
+    first = _prefill_case(Cfg(head_dim=64), pre, n_q, seed=820 + pre, kv=_uneven_rows)[0]
+    again = _prefill_case(Cfg(head_dim=64), pre, n_q, seed=820 + pre, kv=_uneven_rows)[0]
+    np.testing.assert_array_equal(first, again)
+
+
 def _chunk(cfg, pre, n_q, seed, edit=None, sel=False, q_batch=None):
     """Output of a chunk over seeded rows (a row of the chunk's V changed by `edit`)."""
     c = cfg_of(cfg)
