@@ -270,7 +270,7 @@ hipError_t launch_prefill_index(const Geo &g, const qwfn_kv_view &v, const float
 bool pf_approx_fits_shape(int32_t hd, int32_t G);
 hipError_t launch_pf_approx_scores(const Geo &g, const qwfn_kv_view &v, const float *q, int32_t n_q,
                                    int32_t n_blk, float *scores, int32_t nb_cap, float *pnorm, hipStream_t st);
-// The largest q8_0 V scale of each KV head over positions [0, n_pos) of
+// The largest finite V scale of each KV head over positions [0, n_pos) of
 // sequence g.pf_seq, as kVmaxWg partial maxima per head (vmax).
 hipError_t launch_prefill_vmax(const Geo &g, const qwfn_kv_view &v, int32_t n_pos, float *vmax, hipStream_t st);
 // Compute units of the current device (looked up once per device).

@@ -2743,8 +2743,9 @@ __device__ __forceinline__ void wave_lds_sync() {
 }
 
 
-// grid (kVmaxWg, Hkv), 256 threads: partial maxima of KV head gh's q8_0 V
-// scales over positions [0, n_pos) of sequence pf_seq, each a 64-cell tile's
+// grid (kVmaxWg, Hkv), 256 threads: partial maxima of KV head gh's finite V
+// scales (an infinite one would set the unit of every query's values, those
+// before its row too) over positions [0, n_pos) of sequence pf_seq, each a 64-cell tile's
 // scale row read as 16-byte chunks (cell c's NJ scales are halfs c*NJ ..
 // c*NJ+NJ-1 of the row); cells at or past n_pos and unmapped pages are left
 // out.  vmax[gh * kVmaxWg + blockIdx.x] gets the workgroup's maximum.
@@ -2765,7 +2766,7 @@ k_pf_vmax(Geo g, qwfn_kv_view v, int32_t n_pos, float *__restrict__ vmax) {
         const h8v x = __builtin_bit_cast(h8v, w);
 #pragma unroll
         for (int e = 0; e < 8; ++e)
-            if (t0 + (8 * c + e) / NJ < n_pos) mx = fmaxf(mx, fabsf((float)x[e]));
+            if (t0 + (8 * c + e) / NJ < n_pos && fabsf((float)x[e]) < INFINITY) mx = fmaxf(mx, fabsf((float)x[e]));
     }
     mx = wave_max(mx);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = mx;

@@ -219,13 +219,13 @@ k_pf_full(Geo g, qwfn_kv_view v, const float *__restrict__ q, int32_t n_q, const
             }
         lscale[ct] = qs * g.scale_log2;
     }
-    // 2^kv brings the head's largest V value below 2^15 (|quant| <= 128)
+    // 2^kv brings the head's largest finite V value below 2^15 (|quant| <= 128)
     float v_up = 1.0f, v_down = 1.0f;
     if constexpr (C::SCALED) {
         const float dvm = wave_max(vmax[gh * kVmaxWg + l % kVmaxWg]);
         int e2 = 0;
         frexpf(dvm, &e2);
-        if (dvm > 0.0f && dvm < INFINITY) {
+        if (dvm > 0.0f) {
             v_up = ldexpf(1.0f, kFullVTop - 7 - e2);
             v_down = ldexpf(1.0f, e2 + 7 - kFullVTop);
         }

@@ -116,3 +116,31 @@ def test_prefill_every_block_non_finite_rows(kv_type, bad):
     assert not np.isfinite(got[bad:, G:, dims]).any()
     got[bad:, G:, dims], ref[bad:, G:, dims] = 0.0, 0.0
     assert_close_attn(got, ref.astype(np.float64))
+
+
+@pytest.mark.parametrize("kv_type, unit", [(0, 1.0), (0, 1e-3), (0, 5e3), (1, 1.0), (1, 1e-3), (1, 5e3), (2, 1.0), (2, 1e-3)])
+@pytest.mark.parametrize("n_q, bad", [(576, 300), (576, 575), (576, 511), (90, 511), (90, 575)])
+def test_prefill_before_a_non_finite_row(kv_type, unit, n_q, bad):
+    """The queries before a non-finite V row give the bytes of a cache where it holds
+    zeros, in the kernel of a block of queries (576) and of one query (90): the largest V
+    scale of a call, which sets the unit that the values (or weights) are split in, is
+    the largest finite one.  Rows far below 1, and rows past fp16's largest value (at 5e3
+    a quantized block's scale still fits)."""
+    cfg = Cfg(kv_type=kv_type)
+    pre = 576 - n_q
+    dims = slice(32, 64) if kv_type != 2 else slice(40, 41)
+
+    def edit(v):
+        v *= unit
+        v[bad, 1, 40] = np.inf
+
+    def zero(v):
+        v *= unit
+        v[bad, 1, dims] = 0.0
+
+    got, ref = _chunk(cfg, pre, n_q, 92, edit), _chunk(cfg, pre, n_q, 92, zero)
+    np.testing.assert_array_equal(got[:bad - pre], ref[:bad - pre])
+    G, at = cfg.n_head // cfg.n_head_kv, slice(bad - pre, None)
+    assert not np.isfinite(got[at, G:, dims]).any()
+    got[at, G:, dims], ref[at, G:, dims] = 0.0, 0.0
+    assert_close_attn(got[at] / unit, ref[at].astype(np.float64) / unit)
