@@ -608,6 +608,13 @@ int qwfn_sparse_attn_decode_chain(const qwfn_qsa_shape *shape, const qwfn_kv_vie
     int32_t group = 1;
     if (chain_together(g, shape, n_seq, n_pos, max_seq_len))
         for (group = n_pos; group > 1 && decode_ws_bytes(g, shape, group * n_seq, max_seq_len) > ws_bytes;) --group;
+    // position k's lengths: seq_len + k, of the positions that go out together or, one
+    // after the other, of all of them in one launch (the first one alone reads seq_len
+    // itself)
+    if (group == 1 && n_pos > 1) {
+        e = launch_chain_lens(seq_len, n_seq, 0, n_pos, max_seq_len, w.lens, st);
+        if (e != hipSuccess) return hip_fail(e, "decode: chain lengths");
+    }
     for (int32_t k = 0; k < n_pos; k += group) {
         const int32_t np = std::min(group, n_pos - k), rows = np * n_seq;
         const bool many = np > 1;
@@ -618,9 +625,8 @@ int qwfn_sparse_attn_decode_chain(const qwfn_qsa_shape *shape, const qwfn_kv_vie
         } else if (group > 1) {
             if ((rc = bind_ws(g, n_seq, max_seq_len, msel, ws, ws_bytes, &w))) return rc;
         }
-        // position k's lengths: seq_len + k (the first position alone reads seq_len itself)
-        const int32_t *len_k = seq_len;
-        if (many || k > 0) {
+        const int32_t *len_k = group == 1 && k > 0 ? w.lens + (size_t)k * n_seq : seq_len;
+        if (group > 1) {
             e = launch_chain_lens(seq_len, n_seq, k, np, max_seq_len, w.lens, st);
             if (e != hipSuccess) return hip_fail(e, "decode: chain lengths");
             len_k = w.lens;

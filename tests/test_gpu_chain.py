@@ -12,6 +12,8 @@ reading through the writes of the ones before).
 * Captured in one hipGraph: every replay (with eager work between) equals the
   eager chain.
 """
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -209,3 +211,42 @@ def test_chain_groups_equal_single_calls(cfg, lengths, n_pos, part):
     assert qsa.read_status(dev) == qsa.read_status(twin) != 0
     for name in ("k_pages", "v_pages", "pooled"):
         assert torch.equal(getattr(dev, name), getattr(twin, name)), name
+
+
+def _graph_nodes(fn):
+    """Launches `fn` (a call on the current stream) captures into a HIP graph."""
+    with open("/proc/self/maps") as f:
+        path = next(line.split()[-1] for line in f if "libamdhip64" in line)
+    hip = ctypes.CDLL(path)
+    g = torch.cuda.CUDAGraph(keep_graph=True)
+    st = torch.cuda.Stream()
+    st.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(st):
+        with torch.cuda.graph(g, stream=st):
+            fn()
+    n = ctypes.c_size_t(0)
+    assert hip.hipGraphGetNodes(ctypes.c_void_p(g.raw_cuda_graph()), None, ctypes.byref(n)) == 0
+    return n.value
+
+
+@pytest.mark.parametrize("cfg,n_seq,part", [
+    (Cfg(top_k_blocks=0), 1, 1), (Cfg(local_tokens=2), 2, 1),        # nothing to select; too short a window
+    (BASELINE, 9, 1), (BASELINE, 2, 8),                              # many sequences; a workspace for one position
+])
+def test_chain_position_by_position_derives_lengths_once(cfg, n_seq, part):
+    """Where the positions of a chain go out one after the other, all their lengths
+    come from one launch: a chain of 6 is 6 single calls' launches and one more."""
+    lengths, n_pos = [64 * 80 - 3 - 5 * i for i in range(n_seq)], 6
+    print(f"chain launches: {n_seq} sequences, workspace / {part}", flush=True)
+    _, dev, _, q, kn, vn = _setup(cfg, lengths, n_pos, seed=6)
+    c = cfg_of(cfg)
+    cur = torch.tensor(lengths, dtype=torch.int32, device="cuda") + 1
+    max_len = int(cur.max()) + n_pos - 1
+    ws = qsa.Workspace(c, n_seq, max_len, nbytes=-(-c.workspace_bytes(n_seq, max_len) // part // 256) * 256 + 65536)
+    qd, knd, vnd = torch.from_numpy(q).cuda(), torch.from_numpy(kn).cuda(), torch.from_numpy(vn).cuda()
+    out = torch.empty((n_pos, n_seq, cfg.n_head, cfg.head_dim), dtype=torch.float32, device="cuda")
+    qsa.sparse_attn_decode_chain(dev, qd, knd, vnd, cur, max_len, ws, out=out)
+    torch.cuda.synchronize()
+    one = _graph_nodes(lambda: qsa.sparse_attn_decode(dev, qd[0], knd[0], vnd[0], cur, max_len, ws, out=out[0]))
+    chain = _graph_nodes(lambda: qsa.sparse_attn_decode_chain(dev, qd, knd, vnd, cur, max_len, ws, out=out))
+    assert chain == n_pos * one + 1
