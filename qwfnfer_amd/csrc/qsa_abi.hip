@@ -828,7 +828,10 @@ int prefill_impl(const qwfn_qsa_shape *shape, const qwfn_kv_view *view, const Id
     }
     // the leading queries that attend every block up to their position share
     // tiles and need no selection (their batch size is not the workspace's)
-    const int32_t n_full = parts ? 0 : pf_full_queries(gp, pos0, n_q);
+    // (a selection that none of them needs: the bounded scoring's two launches, or
+    // the general indexer of a shape without them)
+    const float sel_us = g.topk <= 0 || sel_out ? 0.0f : ix || pf_approx_fits_shape(g.hd, g.G) ? 12.0f : 300.0f;
+    const int32_t n_full = parts ? 0 : pf_full_queries(gp, pos0, n_q, sel_us);
     if (n_full > 0) {
         gp.pf_pos0 = pos0;
         e = launch_prefill_full(gp, *view, q, n_full, w.vmax, out, st);

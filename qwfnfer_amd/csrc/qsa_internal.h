@@ -284,9 +284,11 @@ hipError_t launch_prefill_attention(const Geo &g, const qwfn_kv_view &v, const f
                                     float *out, hipStream_t st);
 // Prefill attention of queries that attend every block up to their position,
 // a block of queries sharing each tile (qsa_prefill_full.hip).
-// pf_full_queries: how many leading queries of a call do (0 for a shape
-// without an instance); vmax from launch_prefill_vmax (unused for F16).
-int32_t pf_full_queries(const Geo &g, int32_t pos0, int32_t n_q);
+// pf_full_queries: how many leading queries of a call go this way (0 for a shape
+// without an instance, or where the per-query kernels are faster); sel_us: what a
+// call without them spends on a selection that it then does not need.
+// vmax from launch_prefill_vmax (unused for F16).
+int32_t pf_full_queries(const Geo &g, int32_t pos0, int32_t n_q, float sel_us);
 hipError_t launch_prefill_full(const Geo &g, const qwfn_kv_view &v, const float *q, int32_t n_q, const float *vmax,
                                float *out, hipStream_t st);
 // Batched decode attention over a given selection (or every block, sel NULL) with

@@ -704,23 +704,68 @@ int full_layout(const Geo &g) {
 
 }  // namespace
 
-// Measured against the per-query kernels (us a call, whole calls of 2 KV heads;
-// per-query kernel / this one).  A workgroup here walks its tiles in series, 5 us a
-// step of two tiles, so a call of few queries is better split over them:
-//   q8_0, 16 x 128:  203 after 4,000 tokens 103 / 189, 500 after 4,000 176 / 204,
-//     500 from 0 52 / 49, 1,000 from 0 97 / 70, 3,001 from 0 403 / 155, 4,700 from 0
-//     866 / 309, dense 2,000 after 8,000 1,135 / 418;
-//   the K layouts, whose per-query kernel does not split a query: q4_0 200 after
-//     4,000 141 / 208, 3,000 from 0 462 / 166, F16 3,000 from 0 427 / 162, the
-//     checkpoint layer 400 after 1,000 151 / 140, 1,900 from 0 405 / 308.
-constexpr int64_t kFullPairs = 1024, kFullPairsK = 768;   // (query, KV head) pairs from which it is used
+// Measured against the per-query kernels (us a call, whole calls of 2 KV heads on
+// 256 CUs; per-query kernel / this one).  A workgroup here walks its tiles in series, 5
+// us a step of two tiles, so a call of few queries is better split over them.
+//   q8_0, whose per-query kernel splits a query over waves while a call leaves CUs
+//     idle: 16 x 128 dense 512 after 9,000 tokens 306 / 396, 520 388 / 398, 700 455 /
+//     405, 1,000 611 / 418, 3,001 from 0 403 / 155; 16 x 64 dense 512 after 9,000 191 /
+//     244, 520 244 / 244; 16 x 256 512 after 9,000 796 / 662, 24 x 256 925 / 672.  The
+//     line is where that kernel stops sharing pairs: past four a CU, at 256 dims (half
+//     the waves a CU) from four.
+//   The K layouts' per-query kernel (k_dec_loop) is a workgroup a pair whose time goes
+//     in steps with the workgroups a CU, and a call whose every query attends every
+//     block also saves its selection here, so the line moves with the length: dense F16
+//     512 after 9,000 368 / 441, 520 469 / 441, 700 from 0 49 / 50, 1,000 75 / 65; dense
+//     q4_0 512 from 0 38 / 50, 1,000 81 / 75, 512 after 1,500 109 / 118, 600 130 / 124,
+//     512 after 15,000 725 / 700; the checkpoint layer 384 after 1,000 130 / 138, 450
+//     158 / 142, 1,000 329 / 264.  Both sides' times are estimated.
+constexpr int64_t kFullPairsCu = 4, kFullPairsCuK = 3;    // (query, KV head) pairs a CU: the lines (K: no fewer)
 
-int32_t pf_full_queries(const Geo &g, int32_t pos0, int32_t n_q) {
+// What the estimates are made of, us: this kernel's start and its time a tile, and
+// k_dec_loop's time a tile, a part of its own and a part for each pair a CU.
+// Fitted over 240 calls of 1, 2 and 8 KV heads, 64 to 2,000 queries after 0 to 30,000
+// tokens: the side taken is the faster one or within 8% of it in all but eight.
+struct FullCost { float full0, full, loop, loop_cu; };
+constexpr FullCost kFullCostQ8K = {23.0f, 4.95f, 0.6f, 1.15f}, kFullCostQ4 = {28.0f, 2.8f, 0.5f, 0.62f},
+                   kFullCostF16 = {18.0f, 2.86f, 0.1f, 0.58f};
+constexpr float kLoop0 = 14.0f;          // k_dec_loop's start
+
+// This kernel over n queries from position pos0, `wgs` workgroups, the longest first:
+// the rounds before the last one at the mean length of theirs, the last one at its own.
+float full_us(const FullCost &c, int64_t pos0, int64_t n, int64_t wgs) {
+    const int64_t cus = device_cus(), rounds = (wgs + cus - 1) / cus;
+    const float t = (float)((pos0 + n + 63) / 64), t0 = (float)(pos0 / 64);
+    const float before = (float)((rounds - 1) * cus) / (float)wgs;
+    const float walk = (float)(rounds - 1) * (t - (t - t0) * before * 0.5f) + t0 + (t - t0) * (1.0f - before) * 0.5f;
+    return c.full0 + c.full * std::max(t, rounds > 1 ? walk : 0.0f);
+}
+
+// k_dec_loop over `pairs` of tiles t0 .. t: up to four workgroups a CU side by side, the
+// ones after them at the mean length.
+float loop_us(const FullCost &c, int64_t pairs, int64_t pos0, int64_t end) {
+    if (pairs <= 0) return 0.0f;
+    const int64_t cus = device_cus(), a_cu = (pairs + cus - 1) / cus;
+    const float t = (float)((end + 63) / 64), t0 = (float)(pos0 / 64);
+    return kLoop0 + t * (c.loop + c.loop_cu * (float)std::min<int64_t>(a_cu, 4)) +
+           c.loop_cu * (float)std::max<int64_t>(a_cu - 4, 0) * 0.5f * (t0 + t);
+}
+
+int32_t pf_full_queries(const Geo &g, int32_t pos0, int32_t n_q, float sel_us) {
     const int ly = full_layout(g);
     if (ly < 0) return 0;
     const int64_t most = g.topk <= 0 ? (int64_t)pos0 + n_q : all_kept_len(g);
     const int64_t n = std::max<int64_t>(0, std::min<int64_t>(n_q, most - pos0));
-    return n * g.Hkv >= (ly == kPlQ8 ? kFullPairs : kFullPairsK) ? (int32_t)n : 0;
+    const int64_t pairs = n * g.Hkv, cus = device_cus();
+    if (ly == kPlQ8) return pairs > kFullPairsCu * cus - (g.hd > 128 ? 1 : 0) ? (int32_t)n : 0;
+    if (pairs < kFullPairsCuK * cus) return 0;
+    const FullCost &c = ly == kPlQ8K ? kFullCostQ8K : ly == kPlQ4 ? kFullCostQ4 : kFullCostF16;
+    const int qb = (g.hd > 128 ? 64 : 128) / g.G;          // FullCfg's queries a workgroup
+    // a call's other queries (they attend a selection) take k_dec_loop either way
+    const int64_t rest = (int64_t)n_q - n, end = std::min((int64_t)pos0 + n_q, most);
+    const float full = full_us(c, pos0, n, (n + qb - 1) / qb * g.Hkv) + loop_us(c, rest * g.Hkv, end, end);
+    const float loop = loop_us(c, (int64_t)n_q * g.Hkv, pos0, end) + (rest == 0 ? sel_us : 0.0f);
+    return full <= loop ? (int32_t)n : 0;
 }
 
 hipError_t launch_prefill_full(const Geo &g, const qwfn_kv_view &v, const float *q, int32_t n_q, const float *vmax,

@@ -2,6 +2,8 @@
 filled with the same seeded rows."""
 from __future__ import annotations
 
+import ctypes
+
 import numpy as np
 import torch
 
@@ -157,3 +159,19 @@ def decode_steps(cfg, lengths, steps, seed, dtype=np.float32, zero_pooled=False,
         nw = int(cur[s]) // cfg.block_tokens
         np.testing.assert_array_equal(np_of(dev.pooled)[s, :, :nw], host.pooled[s, :, :nw])
     return outs
+
+
+def graph_nodes(fn):
+    """Launches `fn` (a call on the current stream) captures into a HIP graph."""
+    with open("/proc/self/maps") as f:
+        path = next(line.split()[-1] for line in f if "libamdhip64" in line)
+    hip = ctypes.CDLL(path)
+    g = torch.cuda.CUDAGraph(keep_graph=True)
+    st = torch.cuda.Stream()
+    st.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(st):
+        with torch.cuda.graph(g, stream=st):
+            fn()
+    n = ctypes.c_size_t(0)
+    assert hip.hipGraphGetNodes(ctypes.c_void_p(g.raw_cuda_graph()), None, ctypes.byref(n)) == 0
+    return n.value

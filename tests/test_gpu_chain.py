@@ -12,13 +12,11 @@ reading through the writes of the ones before).
 * Captured in one hipGraph: every replay (with eager work between) equals the
   eager chain.
 """
-import ctypes
-
 import numpy as np
 import pytest
 import torch
 
-from _gpu import assert_close_attn, cfg_of, fill, kv_rows, make_pair, np_of
+from _gpu import assert_close_attn, cfg_of, fill, graph_nodes, kv_rows, make_pair, np_of
 from _refs import BASELINE, Cfg
 from qwfnfer_amd import qsa
 
@@ -213,22 +211,6 @@ def test_chain_groups_equal_single_calls(cfg, lengths, n_pos, part):
         assert torch.equal(getattr(dev, name), getattr(twin, name)), name
 
 
-def _graph_nodes(fn):
-    """Launches `fn` (a call on the current stream) captures into a HIP graph."""
-    with open("/proc/self/maps") as f:
-        path = next(line.split()[-1] for line in f if "libamdhip64" in line)
-    hip = ctypes.CDLL(path)
-    g = torch.cuda.CUDAGraph(keep_graph=True)
-    st = torch.cuda.Stream()
-    st.wait_stream(torch.cuda.current_stream())
-    with torch.cuda.stream(st):
-        with torch.cuda.graph(g, stream=st):
-            fn()
-    n = ctypes.c_size_t(0)
-    assert hip.hipGraphGetNodes(ctypes.c_void_p(g.raw_cuda_graph()), None, ctypes.byref(n)) == 0
-    return n.value
-
-
 @pytest.mark.parametrize("cfg,n_seq,part", [
     (Cfg(top_k_blocks=0), 1, 1), (Cfg(local_tokens=2), 2, 1),        # nothing to select; too short a window
     (BASELINE, 9, 1), (BASELINE, 2, 8),                              # many sequences; a workspace for one position
@@ -247,6 +229,6 @@ def test_chain_position_by_position_derives_lengths_once(cfg, n_seq, part):
     out = torch.empty((n_pos, n_seq, cfg.n_head, cfg.head_dim), dtype=torch.float32, device="cuda")
     qsa.sparse_attn_decode_chain(dev, qd, knd, vnd, cur, max_len, ws, out=out)
     torch.cuda.synchronize()
-    one = _graph_nodes(lambda: qsa.sparse_attn_decode(dev, qd[0], knd[0], vnd[0], cur, max_len, ws, out=out[0]))
-    chain = _graph_nodes(lambda: qsa.sparse_attn_decode_chain(dev, qd, knd, vnd, cur, max_len, ws, out=out))
+    one = graph_nodes(lambda: qsa.sparse_attn_decode(dev, qd[0], knd[0], vnd[0], cur, max_len, ws, out=out[0]))
+    chain = graph_nodes(lambda: qsa.sparse_attn_decode_chain(dev, qd, knd, vnd, cur, max_len, ws, out=out))
     assert chain == n_pos * one + 1

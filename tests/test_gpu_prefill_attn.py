@@ -5,7 +5,7 @@ import pytest
 import torch
 
 from _ckpt import CKPT
-from _gpu import assert_close_attn, cfg_of, kv_rows, np_of
+from _gpu import assert_close_attn, cfg_of, graph_nodes, kv_rows, np_of
 from _refs import BASELINE, Cfg
 from qwfnfer_amd import qsa
 from test_gpu_parity import _prefill_case
@@ -40,6 +40,38 @@ def test_prefill_few_queries(cfg, pre, n_q):
 ])
 def test_prefill_every_block(cfg, pre, n_q):
     _prefill_case(cfg, pre, n_q, seed=800 + n_q, dtype=np.float16 if n_q % 2 else np.float32)
+
+
+# The same layouts at counts that take the shared pass when the selection is asked for
+# too, and 16 queries more than one round of the per-query kernel.
+@pytest.mark.parametrize("cfg, pre, n_q", [
+    (Cfg(kv_type=1), 5, 1130), (Cfg(kv_type=2), 63, 1051), (Cfg(kv_type=2, block_tokens=16, top_k_blocks=300), 1, 1040),
+    (CKPT, 129, 700), (BASELINE, 0, 528),
+])
+def test_prefill_every_block_longer(cfg, pre, n_q):
+    _prefill_case(cfg, pre, n_q, seed=840 + n_q)
+
+
+@pytest.mark.parametrize("cfg, pre, n_q, shared", [
+    (Cfg(top_k_blocks=0), 900, 512, False), (Cfg(top_k_blocks=0), 900, 513, True),
+    (Cfg(top_k_blocks=0, n_head=8), 900, 512, False), (Cfg(top_k_blocks=0, head_dim=256), 900, 512, True),
+    (Cfg(top_k_blocks=0, kv_type=2), 8000, 500, False), (Cfg(top_k_blocks=0, kv_type=2), 8000, 600, True),
+    (Cfg(top_k_blocks=0, kv_type=2), 0, 520, False), (Cfg(top_k_blocks=0, kv_type=2), 0, 1100, True),
+    (Cfg(kv_type=2), 0, 400, True), (Cfg(kv_type=2), 3500, 400, False), (Cfg(kv_type=2), 3500, 700, True),
+    (Cfg(top_k_blocks=0, kv_type=1), 0, 512, False), (Cfg(top_k_blocks=0, kv_type=1), 0, 1300, True),
+    (Cfg(top_k_blocks=0, kv_type=1), 1500, 500, False), (Cfg(top_k_blocks=0, kv_type=1), 1500, 700, True),
+])
+def test_prefill_every_block_line(cfg, pre, n_q, shared):
+    """Which calls share tiles: those measured faster so (they launch no indexer)."""
+    print(f"line: {n_q} queries after {pre}", flush=True)
+    c = cfg_of(cfg)
+    dev = qsa.KvCache.allocate(c, 1, (pre + n_q) // cfg.page_tokens + 1)
+    rows = torch.zeros((n_q, cfg.n_head_kv, cfg.head_dim), dtype=torch.float16, device="cuda")
+    q, ws = torch.zeros((n_q, cfg.n_head, cfg.head_dim), device="cuda"), qsa.Workspace.for_prefill(c, pre + n_q, n_q)
+    out = torch.empty_like(q)
+    n = graph_nodes(lambda: qsa.sparse_attn_prefill(dev, q, 0, pre, ws, rows, rows, out=out))
+    before = 2 if cfg.kv_type == 2 else 3            # the rows, the pooled keys, the V scales
+    assert (n == before + 1) == shared and n >= before + 1
 
 
 def _uneven_rows(rng, n, cfg):
