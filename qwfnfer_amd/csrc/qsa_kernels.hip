@@ -2833,7 +2833,7 @@ struct PfAttnLds {
 // of them taking tiles u, u + split, ..., and add up their states through LDS at
 // the end (pf_split picks the count).
 // MODE kPfDecode: a batched decode's attention over a given selection (sel) or
-// every block (sel NULL): grid (parts, Hkv, n_seq), kPfDecWaves waves a workgroup,
+// every block (sel NULL): grid (parts, n_seq Hkv), kPfDecWaves waves a workgroup,
 // two workgroups a CU; the waves share tiles [part split, (part + 1) split) of a
 // (sequence, KV head) and leave one partial (max, sum, unnormalised O) for k_merge.
 // There 2^k follows the largest V scale of the tiles a wave has met (a power of
@@ -2856,7 +2856,7 @@ k_pf_attn(Geo g, qwfn_kv_view v, const float *__restrict__ q, int32_t n_q, const
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = threadIdx.x & 63;
     const int nsp = DEC ? WAVES : SPLIT ? split : 1; // waves a pair (divides WAVES)
     const int sub = SPLIT ? wv % nsp : 0;            // this wave's place among them
-    int pair = DEC     ? (int)blockIdx.z * g.Hkv + (int)blockIdx.y
+    int pair = DEC     ? (int)blockIdx.y
                : SPLIT ? (int)blockIdx.x * (WAVES / nsp) + wv / nsp
                        : (int)blockIdx.x * WAVES + wv;
     const bool live = DEC || pair < n_q * g.Hkv;
@@ -2870,7 +2870,10 @@ k_pf_attn(Geo g, qwfn_kv_view v, const float *__restrict__ q, int32_t n_q, const
     const bool hv = hn < G;
     const int tpb = g.bt / 64;
     const int n = DEC && !(L >= 1 && L <= n_q) ? 0 : min(DEC && !sel ? (L - 1) / g.bt + 1 : nsel[pair], max_sel);
-    const int t_first = DEC ? (int)blockIdx.x * split : 0;           // this workgroup's tiles
+    // this workgroup's part (an even count starts each pair's at another one, see
+    // launch_dec_walk) and tiles
+    const int part = !DEC ? 0 : gridDim.x % 2 ? (int)blockIdx.x : (int)((blockIdx.x + blockIdx.y) % gridDim.x);
+    const int t_first = part * split;
     if (DEC && t_first >= n * tpb) return;           // (the whole workgroup) no partial: the merge reads fewer
     const int32_t *selp = sel + (int64_t)pair * max_sel;
     // PAIR (8 heads, head_dim >= 128): QK's 16 columns hold every head twice,
@@ -3283,7 +3286,7 @@ k_pf_attn(Geo g, qwfn_kv_view v, const float *__restrict__ q, int32_t n_q, const
                 t += reinterpret_cast<const f4v *>(&shw[w0 + u].buf[0])[i];
             }
             if constexpr (DEC) {
-                const int64_t pb = ((int64_t)pair * ws.n_tiles + blockIdx.x) * G;
+                const int64_t pb = ((int64_t)pair * ws.n_tiles + part) * G;
                 reinterpret_cast<f4v *>(ws.part_o + pb * HD)[i] = t;
                 if (i % (HD / 4) == 0) *reinterpret_cast<float2 *>(&ws.part_ml[(pb + h) * 2]) = make_float2(mx, ls);
                 continue;
@@ -3374,10 +3377,14 @@ int dec_walk_tiles(const Geo &g, int64_t pairs, int n_tiles) {
 hipError_t launch_dec_walk(const Geo &g, const qwfn_kv_view &v, const float *q, const int32_t *seq_len, int32_t n_seq,
                            int32_t max_seq_len, const int32_t *sel, const int32_t *nsel, int32_t max_sel,
                            const Ws &ws, int32_t tpw, hipStream_t st) {
-    // an odd count of parts: workgroups go to the eight XCDs in turn, and the first parts
-    // of short rows would otherwise meet on the same ones (dense, 32 sequences of 1,000
-    // .. 16,000 tokens: 69.5 us with 32 parts, 47.3 with 33)
-    const dim3 grid((unsigned)((ws.n_tiles + tpw - 1) / tpw) | 1u, (unsigned)g.Hkv, (unsigned)n_seq);
+    // Workgroups go to the eight XCDs in turn.  With an even count of parts the first
+    // parts of every pair, all that short rows have, would meet on the same ones (dense,
+    // 32 sequences of 1,000 .. 16,000 tokens: 69.5 us), so the kernel starts pair p's
+    // parts at part p mod the count (47.8).  An idle part more makes the count odd too
+    // (47.1), but costs parts that fill the device's workgroups another round: 32
+    // sequences of 2,000 tokens 26.1 us with it, 23.1 rotated (k_dec 23.3); 16 of
+    // 1,000 .. 16,000 37.6, 31.0.
+    const dim3 grid((unsigned)((ws.n_tiles + tpw - 1) / tpw), (unsigned)(g.Hkv * n_seq));
 #define X(HD_, G_)                                                                                                  \
     if (g.hd == HD_ && g.G == G_) {                                                                                 \
         QWFN_LAUNCH(kTimedAttention, (k_pf_attn<HD_, G_, kPfDecode>), grid, dim3(kPfDecWaves * 64), st, g, v, q,     \

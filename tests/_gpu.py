@@ -161,8 +161,13 @@ def decode_steps(cfg, lengths, steps, seed, dtype=np.float32, zero_pooled=False,
     return outs
 
 
-def graph_nodes(fn):
-    """Launches `fn` (a call on the current stream) captures into a HIP graph."""
+def graph_grids(fn):
+    """Grid (x, y, z) of each kernel that `fn` (a call on the current stream) captures
+    into a HIP graph."""
+    class Params(ctypes.Structure):
+        _fields_ = [("block", ctypes.c_uint * 3), ("extra", ctypes.c_void_p), ("func", ctypes.c_void_p),
+                    ("grid", ctypes.c_uint * 3), ("args", ctypes.c_void_p), ("shared", ctypes.c_uint)]
+
     with open("/proc/self/maps") as f:
         path = next(line.split()[-1] for line in f if "libamdhip64" in line)
     hip = ctypes.CDLL(path)
@@ -172,6 +177,18 @@ def graph_nodes(fn):
     with torch.cuda.stream(st):
         with torch.cuda.graph(g, stream=st):
             fn()
-    n = ctypes.c_size_t(0)
-    assert hip.hipGraphGetNodes(ctypes.c_void_p(g.raw_cuda_graph()), None, ctypes.byref(n)) == 0
-    return n.value
+    raw, n = ctypes.c_void_p(g.raw_cuda_graph()), ctypes.c_size_t(0)
+    assert hip.hipGraphGetNodes(raw, None, ctypes.byref(n)) == 0
+    nodes = (ctypes.c_void_p * n.value)()
+    assert hip.hipGraphGetNodes(raw, nodes, ctypes.byref(n)) == 0
+    grids = []
+    for node in nodes:
+        p = Params()
+        assert hip.hipGraphKernelNodeGetParams(ctypes.c_void_p(node), ctypes.byref(p)) == 0
+        grids.append(tuple(p.grid))
+    return grids
+
+
+def graph_nodes(fn):
+    """Launches `fn` captures into a HIP graph."""
+    return len(graph_grids(fn))

@@ -31,7 +31,7 @@ import numpy as np
 import pytest
 import torch
 
-from _gpu import assert_close_attn, cfg_of, decode_steps, fill, kv_rows, make_pair, np_of
+from _gpu import assert_close_attn, cfg_of, decode_steps, fill, graph_grids, kv_rows, make_pair, np_of
 from _refs import BASELINE, Cfg
 from qwfnfer_amd import qsa
 
@@ -169,6 +169,45 @@ def test_batched_attention_walks_tiles(cfg, lengths):
     workgroup share a part of a sequence's tiles (one, two or more a wave, parts that end
     inside it, empty ones past a short sequence)."""
     decode_steps(cfg, lengths, 1, seed=len(lengths), reattend=True)
+
+
+def _walk_grid(cfg, n_seq, tokens):
+    """Grid of a decode step's attention that walks tiles (parts, (sequence, KV head)), or
+    None where the step launches none."""
+    c = cfg_of(cfg)
+    dev = qsa.KvCache.allocate(c, n_seq, tokens // cfg.page_tokens + 1)
+    q = torch.zeros((n_seq, cfg.n_head, cfg.head_dim), device="cuda")
+    rows = torch.zeros((n_seq, cfg.n_head_kv, cfg.head_dim), device="cuda")
+    lens = torch.full((n_seq,), tokens, dtype=torch.int32, device="cuda")
+    ws, out = qsa.Workspace(c, n_seq, tokens), torch.empty_like(q)
+    step = lambda: qsa.sparse_attn_decode(dev, q, rows, rows, lens, tokens, ws, out=out)
+    step()
+    torch.cuda.synchronize()
+    got = [g for g in graph_grids(step) if g[1:] == (n_seq * cfg.n_head_kv, 1)]
+    return got[0] if got else None
+
+
+@pytest.mark.parametrize("cfg, n_seq, tokens, parts", [
+    (Cfg(top_k_blocks=0), 32, 2048, 8), (Cfg(top_k_blocks=0), 40, 2049, 9), (Cfg(top_k_blocks=0), 64, 2048, 4),
+    (Cfg(top_k_blocks=0, head_dim=64), 24, 12288, 24), (BASELINE, 32, 9000, 10), (BASELINE, 24, 9000, 19),
+])
+def test_batched_attention_launches_no_idle_part(cfg, n_seq, tokens, parts):
+    """As many parts a (sequence, KV head) as its tiles make, odd or even: a part more
+    could cost every call whose parts just fill the device another round."""
+    print(f"parts: {n_seq} sequences of {tokens}, {parts}", flush=True)
+    assert _walk_grid(cfg, n_seq, tokens) == (parts, n_seq * cfg.n_head_kv, 1)
+
+
+@pytest.mark.parametrize("cfg, n_seq, longest", [
+    (Cfg(top_k_blocks=0), 33, 2048), (Cfg(top_k_blocks=0), 20, 8192), (Cfg(top_k_blocks=0, n_head=8), 33, 4097),
+    (Cfg(top_k_blocks=0, head_dim=64), 17, 16384), (BASELINE, 33, 6000),
+])
+def test_batched_attention_parts_start_anywhere(cfg, n_seq, longest):
+    """Even and odd counts of parts, pairs past a multiple of them, sequences that end in
+    their first, a middle and their last part, one cell past it, or hold one token."""
+    print(f"rotated parts: {n_seq} sequences to {longest}", flush=True)
+    lengths = [longest - 1, 0, 255, 256, longest // 2, longest - 64, 63, 1023]
+    decode_steps(cfg, [lengths[i % 8] for i in range(n_seq)], 1, seed=n_seq, reattend=True)
 
 
 def test_batched_attention_wide_v_scales():
