@@ -1796,8 +1796,20 @@ int launch_dec_t(const Geo &g, const qwfn_kv_view &v, const float *q, const int3
     return 4;
 }
 
+// Tiles a CU past which launch_dec_walk is taken; up to there k_dec, two tiles a
+// workgroup, is faster.  us a step, k_dec / walk, dense with equal lengths unless said:
+// 8 heads a KV head: 4.5 tiles a CU (12 sequences of 188 .. 3,000 tokens) 16.6 / 18.0,
+// 6 (16 of 3,000) 19.3 / 20.0, 6 (24 of 2,000) 20.2 / 21.5; 6.8 (12 of 4,500) 21.3 /
+// 20.8, 9 (16 of 4,500) 24.6 / 26.7, but 20.0 / 19.3 with lengths down to 281.  4 heads,
+// whose k_dec does less a tile: 9 (16 of 4,500) 23.3 / 26.0, 9.3 (16 of 16,000, 74
+// blocks kept) 30.3 / 33.1; 12 (32 of 3,000) 26.2 / 28.0, but 21.0 / 18.4 with lengths
+// down to 188, 16 (16 of 8,000) 32.6 / 31.8.  64 dims: the device holds more than six a
+// CU of k_dec.
+template <int HD, int G> constexpr int dec_walk_cu() { return HD != 128 ? 0 : G == 8 ? 6 : 10; }
+
 // Whether a given-selection or dense q8_0 call goes to launch_dec_walk: when its
-// tiles, one a workgroup, are more than the device holds of k_dec at once.
+// tiles, one a workgroup, are more than the device holds of k_dec at once and past
+// dec_walk_cu.
 template <int HD, int G>
 bool dec_walk_pays(const Geo &g, int32_t n_seq, int32_t max_seq_len, bool given, const Ws &ws) {
     const int npt_lds = dec_npt_lds(g, max_seq_len, given ? kGiven : kDense);
@@ -1805,7 +1817,8 @@ bool dec_walk_pays(const Geo &g, int32_t n_seq, int32_t max_seq_len, bool given,
                                   dec_union_bytes<HD, G, kGiven, 1, kLyQ8>() + 4 * npt_lds)
                             : dec_resident<HD, G, kDense, 4, 1, false, kLyQ8>(
                                   dec_union_bytes<HD, G, kDense, 1, kLyQ8>() + 4 * npt_lds);
-    return r > 0 && (int64_t)(g.chain ? g.chain : n_seq) * g.Hkv * ws.n_tiles > r;
+    const int64_t tiles = (int64_t)(g.chain ? g.chain : n_seq) * g.Hkv * ws.n_tiles;
+    return r > 0 && tiles > r && tiles > (int64_t)dec_walk_cu<HD, G>() * device_cus();
 }
 
 template <int HD, int G, bool RF, int LY>

@@ -3361,12 +3361,12 @@ static void launch_pf_attn_t(const Geo &g, const qwfn_kv_view &v, const float *q
 
 // One tile a wave while the call's tiles (at most) are under two rounds of the device's
 // waves, else two, and at most 96 parts a row, which the merge reads on a workgroup
-// a head.  Measured, us a step (k_dec; parts of 4, by this rule, of 12 tiles): 32
-// sequences of 1,000 .. 40,000 tokens 39.8; 39.8, 39.2, 40.2 (35.5 by the rule in another
-// run), 32 of 40,000 49.1; 50.8, 50.7, 46.5, 16 of 1,000 .. 160,000 30.1; 30.5, 30.5, 32.6;
-// dense, 32 of 1,000 .. 16,000 61.3; 52.6, 47.3, 43.9, 16 of 16,000 55.1; 54.7, 47.6, 46.9,
-// 16 of 1,000 .. 16,000 37.0; 32.0, 30.7, 33.0, one of 100,000 43.4; 30.7, 30.6, 30.4 (of 4
-// tiles without the bound 43.4).
+// a head.  No length of part is best throughout: of equal lengths long parts gain, of
+// mixed ones short parts.  Dense, us a step (k_dec; parts of 4, 8, 12, 16 tiles): 24
+// sequences of 4,500 tokens 31.1; 32.9, 29.5, 32.8, 28.4, of 281 .. 4,500 24.9; 21.4, 24.8,
+// 29.0, 26.9; 16 of 8,000 35.9; 35.2, 32.4, 35.2, 31.2; 32 of 500 .. 8,000 44.0; 35.5, 30.9,
+// 34.5, 36.4; 32 of 16,000 99.6; 105.8, 80.3, 78.9, 73.9, of 1,000 .. 16,000 59.5; 52.7, 48.0,
+// 50.0, 43.7.  One of 100,000: 43.4; of 4 without the bound 43.4, with it (20) 30.7.
 int dec_walk_tiles(const Geo &g, int64_t pairs, int n_tiles) {
     const int64_t waves = 2 * (int64_t)device_cus() * kPfDecWaves;
     const int64_t per = std::min<int64_t>(2, pairs * n_tiles / waves);

@@ -198,6 +198,18 @@ def test_batched_attention_launches_no_idle_part(cfg, n_seq, tokens, parts):
     assert _walk_grid(cfg, n_seq, tokens) == (parts, n_seq * cfg.n_head_kv, 1)
 
 
+@pytest.mark.parametrize("cfg, n_seq, tokens, walks", [
+    (Cfg(top_k_blocks=0), 24, 2048, False), (Cfg(top_k_blocks=0), 25, 2048, True),      # 6 tiles a CU of 256
+    (Cfg(top_k_blocks=0), 12, 3000, False), (BASELINE, 10, 6000, False), (BASELINE, 11, 6000, True),
+    (Cfg(top_k_blocks=0, n_head=8), 20, 4096, False), (Cfg(top_k_blocks=0, n_head=8), 21, 4096, True),     # 10
+    (Cfg(n_head=8), 16, 16000, False), (Cfg(n_head=8), 18, 16000, True),
+])
+def test_batched_attention_line(cfg, n_seq, tokens, walks):
+    """Which batches walk their tiles: those whose tiles a CU were measured faster so."""
+    print(f"line: {n_seq} sequences of {tokens}", flush=True)
+    assert (_walk_grid(cfg, n_seq, tokens) is not None) == walks
+
+
 @pytest.mark.parametrize("cfg, n_seq, longest", [
     (Cfg(top_k_blocks=0), 33, 2048), (Cfg(top_k_blocks=0), 20, 8192), (Cfg(top_k_blocks=0, n_head=8), 33, 4097),
     (Cfg(top_k_blocks=0, head_dim=64), 17, 16384), (BASELINE, 33, 6000),
