@@ -160,6 +160,18 @@ def test_python_errors_carry_the_message():
     assert ei.value.code == _lib.QWFN_EINVAL and "n_head" in str(ei.value)
 
 
+def test_current_stream_without_the_private_handle(monkeypatch):
+    """The current stream's handle also under a torch without its private function."""
+    class Stream:
+        cuda_stream = 77
+
+    monkeypatch.setattr(qsa.torch.cuda, "is_initialized", lambda: True)
+    monkeypatch.setattr(qsa.torch.cuda, "current_stream", lambda: Stream)
+    monkeypatch.delattr(qsa.torch._C, "_cuda_getCurrentRawStream", raising=False)
+    assert qsa._stream(None) == 77
+    assert qsa._stream(5) == 5
+
+
 def test_prefill_rejects_bad_arguments_before_launch():
     cfg = QsaConfig()
     s = cfg.shape()
