@@ -115,12 +115,12 @@ def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
 
 def _stream(stream) -> int:
     if stream is None:
-        # the same handle without the Stream object, where this torch has the function (it
-        # is no part of torch's public interface)
-        raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
-        if raw is None or not torch.cuda.is_initialized():
-            return torch.cuda.current_stream().cuda_stream
-        return raw(torch.cuda.current_device())
+        if torch.cuda.is_initialized():
+            try:                                   # the same handle without the Stream object
+                return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+            except AttributeError:                 # (neither is part of torch's public interface)
+                pass
+        return torch.cuda.current_stream().cuda_stream
     if isinstance(stream, torch.cuda.Stream):
         return stream.cuda_stream
     return int(stream)
