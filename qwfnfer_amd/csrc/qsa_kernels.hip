@@ -3379,12 +3379,16 @@ hipError_t launch_dec_walk(const Geo &g, const qwfn_kv_view &v, const float *q, 
                            const Ws &ws, int32_t tpw, hipStream_t st) {
     // Workgroups go to the eight XCDs in turn.  With an even count of parts the first
     // parts of every pair, all that short rows have, would meet on the same ones (dense,
-    // 32 sequences of 1,000 .. 16,000 tokens: 69.5 us), so the kernel starts pair p's
-    // parts at part p mod the count (47.8).  An idle part more makes the count odd too
-    // (47.1), but costs parts that fill the device's workgroups another round: 32
-    // sequences of 2,000 tokens 26.1 us with it, 23.1 rotated (k_dec 23.3); 16 of
-    // 1,000 .. 16,000 37.6, 31.0.
-    const dim3 grid((unsigned)((ws.n_tiles + tpw - 1) / tpw), (unsigned)(g.Hkv * n_seq));
+    // 32 sequences of 1,000 .. 16,000 tokens: 69.5 us).  An idle part more makes the
+    // count odd (47.1), where it starts no further round of workgroups on the CUs; else
+    // the kernel starts pair p's parts at part p mod the count (47.8).  32 sequences of
+    // 2,000 tokens, 512 workgroups: 26.1 us with the idle parts, 23.1 rotated (k_dec
+    // 23.3), 16 of 1,000 .. 16,000 37.6, 31.0; 32 of 1,000 .. 40,000, 74 blocks kept, 640
+    // workgroups: 36.6, 37.6.
+    const int64_t pairs = (int64_t)g.Hkv * n_seq, cus = device_cus();
+    int64_t parts = (ws.n_tiles + tpw - 1) / tpw;
+    if (parts % 2 == 0 && (pairs * (parts + 1) + cus - 1) / cus == (pairs * parts + cus - 1) / cus) ++parts;
+    const dim3 grid((unsigned)parts, (unsigned)pairs);
 #define X(HD_, G_)                                                                                                  \
     if (g.hd == HD_ && g.G == G_) {                                                                                 \
         QWFN_LAUNCH(kTimedAttention, (k_pf_attn<HD_, G_, kPfDecode>), grid, dim3(kPfDecWaves * 64), st, g, v, q,     \

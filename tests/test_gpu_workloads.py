@@ -188,12 +188,13 @@ def _walk_grid(cfg, n_seq, tokens):
 
 
 @pytest.mark.parametrize("cfg, n_seq, tokens, parts", [
-    (Cfg(top_k_blocks=0), 32, 2048, 8), (Cfg(top_k_blocks=0), 40, 2049, 9), (Cfg(top_k_blocks=0), 64, 2048, 4),
-    (Cfg(top_k_blocks=0, head_dim=64), 24, 12288, 24), (BASELINE, 32, 9000, 10), (BASELINE, 24, 9000, 19),
+    (Cfg(top_k_blocks=0), 32, 2048, 8), (Cfg(top_k_blocks=0), 64, 2048, 4),         # a part more: a round more
+    (Cfg(top_k_blocks=0), 40, 2049, 9), (BASELINE, 24, 9000, 19),                   # odd
+    (Cfg(top_k_blocks=0, head_dim=64), 24, 12288, 25), (BASELINE, 32, 9000, 11),    # even, made odd
 ])
-def test_batched_attention_launches_no_idle_part(cfg, n_seq, tokens, parts):
-    """As many parts a (sequence, KV head) as its tiles make, odd or even: a part more
-    could cost every call whose parts just fill the device another round."""
+def test_batched_attention_idle_part_starts_no_round(cfg, n_seq, tokens, parts):
+    """Parts a (sequence, KV head): as many as its tiles make, one idle one more where that
+    makes the count odd and starts no further round of workgroups on 256 CUs."""
     print(f"parts: {n_seq} sequences of {tokens}, {parts}", flush=True)
     assert _walk_grid(cfg, n_seq, tokens) == (parts, n_seq * cfg.n_head_kv, 1)
 
