@@ -423,7 +423,12 @@ int qwfn_qsa_prefill_workspace_bytes(const qwfn_qsa_shape *shape, int32_t max_se
  * The queries are processed in batches sized to ws_bytes (see
  * qwfn_qsa_prefill_workspace_bytes), each batch a scoring, a selection and
  * an attention launch (and the merge of its partials for the general
- * attention kernel) on `stream`. */
+ * attention kernel) on `stream`; leading queries that attend every block may
+ * share an attention launch of their own.
+ * Selections do not depend on the call's size.  The order of a query's sums
+ * does (how the kernels split its tiles follows n_q), so a prompt prefilled in
+ * other chunks gives outputs that differ in fp32 rounding; ws_bytes changes
+ * nothing. */
 int qwfn_sparse_attn_prefill(const qwfn_qsa_shape *shape, const qwfn_kv_view *view,
                              const float *q, const void *k_new, const void *v_new,
                              int32_t src_dtype, int32_t seq, int32_t pos0, int32_t n_q,

@@ -587,10 +587,8 @@ int qwfn_sparse_attn_decode_chain(const qwfn_qsa_shape *shape, const qwfn_kv_vie
     if ((rc = bind_ws(g, n_seq, max_seq_len, msel, ws, ws_bytes, &w))) return rc;
     hipStream_t st = (hipStream_t)stream;
     hipError_t e = hipSuccess;
-    // one or a few sequences: the attention workgroups select for themselves
-    // (no launch between the scores and the attention; at eight sequences a
-    // selection launch of one workgroup per (sequence, KV head) before a
-    // given-selection attention measured 29.4 against 26.9 us a step)
+    // one or a few sequences: the attention workgroups select for themselves (no
+    // launch between the scores and the attention; see kAttnSelSeqs)
     const bool own = attn_select_fits(g, n_seq, max_seq_len, msel);
     // more sequences: scores, then the selections in a launch of their own (one
     // workgroup a (sequence, KV head), started by the stream, where the indexer's

@@ -2392,6 +2392,8 @@ struct RefineBigShared {
 // the longest query's row: the checkpoint's 1,900 queries at 40,003 tokens (10,476
 // blocks) 426 us with 40 a thread, 303 with 12; whole prefill calls of 1,500 queries
 // at 47,000 tokens 944 us, 855, at 90,000 (24 a thread) 1,097, 1,009.
+// 12, 24 and 40 alone: a row just past one of them loads up to twice what it holds, for
+// an instance less of each shape.
 template <int HD, int G, int KPT>
 __global__ void __launch_bounds__(kRbThreads)
 k_pf_refine_big(Geo g, qwfn_kv_view v, const float *__restrict__ q, float *scores, int32_t nb_cap,
@@ -3464,9 +3466,11 @@ hipError_t launch_attention(const Geo &g, const qwfn_kv_view &v, const float *q,
     return hipErrorInvalidValue;
 }
 
-// Up to this many sequences the attention's own selection pays (measured at 1
-// and 8: 21.5 against 23.8 us per layer, and 36.3 against 42.4 us per step of
-// eight); past it the chip fills and the redundant selections would compete.
+// Up to this many sequences the attention selects for itself.  us a step, so / with
+// the selection in a launch of its own, all of 40,000 tokens and 1,000 .. 40,000: one
+// 15.9 / 17.5, 15.3 / 16.5; two 17.5 / 18.6, 17.5 / 18.5; four 21.1 / 21.6, 18.7 / 20.2;
+// six 24.5 / 24.0, 22.3 / 23.2; eight 22.8 / 24.1, 21.7 / 23.0; nine 23.8 / 25.0, 22.3 /
+// 23.8; twelve 27.6 / 28.0, 25.5 / 25.3, where the redundant selections start to cost.
 constexpr int32_t kAttnSelSeqs = 8;
 
 bool attn_select_fits(const Geo &g, int32_t n_seq, int32_t max_seq_len, int32_t max_sel) {

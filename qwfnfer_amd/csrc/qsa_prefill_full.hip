@@ -595,7 +595,7 @@ k_pf_full(Geo g, qwfn_kv_view v, const float *__restrict__ q, int32_t n_q, const
         if (((st + 2) & 63) == 0) look_up(st + 2);
         load_k(st + 2);
         // ---- the matrix half: PV, then the next tile's QK
-        // ---- PV: unit u = (16 dims u / 2, 32 cells u % 2), operands read two units
+        // ---- PV: unit u = (16 dims u / 2, 32 cells u % 2), operands read one unit
         // ahead of their MFMAs
         h8v va[2][C::VP];
         auto read_v = [&](int u) {
