@@ -505,15 +505,18 @@ k_pf_full(Geo g, qwfn_kv_view v, const float *__restrict__ q, int32_t n_q, const
                 read_k(mb, kf);
 #pragma unroll
                 for (int ct = 0; ct < NCT; ++ct) sv[ct][mb] = f4v{0.0f, 0.0f, 0.0f, 0.0f};
+                // the low parts' sum first: a product of the high parts' sums rounds at the
+                // logit's size, one of the low parts' at 2^-11 of it
 #pragma unroll
-                for (int j = 0; j < NJ; ++j) {
-#pragma unroll
-                    for (int ct = 0; ct < NCT; ++ct)
-                        sv[ct][mb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[j], qh[ct][j], sv[ct][mb], 0, 0, 0);
+                for (int j = 0; j < NJ; ++j)
 #pragma unroll
                     for (int ct = 0; ct < NCT; ++ct)
                         sv[ct][mb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[j], ql[ct][j], sv[ct][mb], 0, 0, 0);
-                }
+#pragma unroll
+                for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                    for (int ct = 0; ct < NCT; ++ct)
+                        sv[ct][mb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[j], qh[ct][j], sv[ct][mb], 0, 0, 0);
             }
         }
     };

@@ -176,3 +176,32 @@ def test_prefill_before_a_non_finite_row(kv_type, unit, n_q, bad):
     assert not np.isfinite(got[at, G:, dims]).any()
     got[at, G:, dims], ref[at, G:, dims] = 0.0, 0.0
     assert_close_attn(got[at] / unit, ref[at].astype(np.float64) / unit)
+
+
+def test_prefill_every_block_f16_precision():
+    """F16: the shared pass is no further from 64 bits than the per-query kernel over the
+    same rows (1,100 queries in one call and in calls of 100).  Both round a logit's sums
+    over the high parts four times at its size; summing high and low parts in turn rounded
+    it eight times, sqrt(2) the error; 1.2 lies between."""
+    cfg = Cfg(kv_type=2)
+    pre, n_q, G = 300, 1100, cfg.n_head // cfg.n_head_kv
+    n = pre + n_q
+    rng = np.random.default_rng(21)
+    k, v = (torch.from_numpy(x).cuda().half() for x in kv_rows(rng, n, cfg))
+    q = torch.from_numpy(rng.standard_normal((n_q, cfg.n_head, cfg.head_dim), dtype=np.float32)).cuda()
+    c = cfg_of(cfg)
+    dev = qsa.KvCache.allocate(c, 1, n // cfg.page_tokens + 1)
+    qsa.append_q8_0(dev, k, v, torch.arange(n, dtype=torch.int32, device="cuda"))
+    qsa.pool_rebuild(dev, 0, n // cfg.block_tokens)
+    ws = qsa.Workspace.for_prefill(c, n, n_q)
+    shared = qsa.sparse_attn_prefill(dev, q, 0, pre, ws)
+    single = torch.cat([qsa.sparse_attn_prefill(dev, q[i:i + 100], 0, pre + i, ws) for i in range(0, n_q, 100)])
+    seen = torch.arange(n, device="cuda") <= pre + torch.arange(n_q, device="cuda")[:, None]
+    err = {"shared": 0.0, "single": 0.0}
+    for h in range(cfg.n_head):
+        s = q[:, h].double() @ k[:, h // G].double().T.contiguous() / cfg.head_dim ** 0.5
+        ref = torch.softmax(s.masked_fill(~seen, -float("inf")), 1) @ v[:, h // G].double()
+        for name, out in (("shared", shared), ("single", single)):
+            err[name] += float(((out[:, h].double() - ref) ** 2).sum())
+    print(f"squared errors {err}", flush=True)
+    assert 0.0 < err["shared"] <= 1.2 ** 2 * err["single"]
