@@ -364,10 +364,10 @@ int qwfn_sparse_attn_decode(const qwfn_qsa_shape *shape, const qwfn_kv_view *vie
  * [qwfn_qsa_max_selected] and n_sel_out [n_pos][n_seq][n_head_kv] (optional).
  * max_seq_len bounds seq_len + n_pos - 1.  One small launch derives the
  * lengths of the positions that go out together (of all of them, where they go
- * out in turn) into the workspace.  The positions then go out together, as rows of one scoring, one attention and one merge launch and a pooling of
- * the blocks they complete, as many at a time as the workspace holds, where the
- * attention selects for itself (qwfn_sparse_attn_decode) and local_tokens >=
- * n_pos; else each position makes qwfn_sparse_attn_decode's launches in turn.
+ * out in turn) into the workspace.  The positions then go out together, as rows
+ * of one scoring, one attention and one merge launch and a pooling of the blocks
+ * they complete, as many at a time as the workspace holds, where the attention
+ * selects for itself (qwfn_sparse_attn_decode) and local_tokens >= n_pos; else each position makes qwfn_sparse_attn_decode's launches in turn.
  * The results are the same.  All on `stream`, so the chain captures into one
  * hipGraph.  n_pos = 1 is qwfn_sparse_attn_decode.                            */
 int qwfn_sparse_attn_decode_chain(const qwfn_qsa_shape *shape, const qwfn_kv_view *view,

@@ -135,7 +135,7 @@ __device__ __forceinline__ bool f16_bad(uint32_t half) { return (half & 0x7c00u)
 //  - QK: S[cell][column] = sum_j dk(cell, j) (K_j[cell][:] . q_j[:, column])
 //    with the key quants exact in fp16 and the query, scaled by a power of
 //    two, as fp16 high + low parts: exact products, two MFMAs a 32-dim block,
-//    the block's scale applied in fp32 (F16: no scales, one chain);
+//    the block's scale applied in fp32 (F16: no scales, one chain, the low parts first);
 //  - PV: O[dim][column] += V[dim][cell] P[cell][column] with V = dv q 2^kv and P =
 //    p 2^14 each as fp16 high + low parts, hi hi + hi lo + lo hi (lo lo is below
 //    2^-24 of the product).  Dequantizing V costs an MFMA more than folding
