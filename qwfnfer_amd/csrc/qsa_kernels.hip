@@ -2835,7 +2835,7 @@ struct PfAttnLds {
 // of them taking tiles u, u + split, ..., and add up their states through LDS at
 // the end (pf_split picks the count).
 // MODE kPfDecode: a batched decode's attention over a given selection (sel) or
-// every block (sel NULL): grid (parts, n_seq Hkv), kPfDecWaves waves a workgroup,
+// every block (sel NULL): grid (parts, Hkv, n_seq), kPfDecWaves waves a workgroup,
 // two workgroups a CU; the waves share tiles [part split, (part + 1) split) of a
 // (sequence, KV head) and leave one partial (max, sum, unnormalised O) for k_merge.
 // There 2^k follows the largest V scale of the tiles a wave has met (a power of
@@ -2858,14 +2858,15 @@ k_pf_attn(Geo g, qwfn_kv_view v, const float *__restrict__ q, int32_t n_q, const
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = threadIdx.x & 63;
     const int nsp = DEC ? WAVES : SPLIT ? split : 1; // waves a pair (divides WAVES)
     const int sub = SPLIT ? wv % nsp : 0;            // this wave's place among them
-    int pair = DEC     ? (int)blockIdx.y
+    int pair = DEC     ? (int)(blockIdx.z * g.Hkv + blockIdx.y)
                : SPLIT ? (int)blockIdx.x * (WAVES / nsp) + wv / nsp
                        : (int)blockIdx.x * WAVES + wv;
     const bool live = DEC || pair < n_q * g.Hkv;
     if (!SPLIT && !live) return;                     // a whole wave; no workgroup barrier follows
     if (SPLIT && !live) pair = n_q * g.Hkv - 1;      // (walks no tile and writes nothing)
     PfAttnLds<HD, G> &W = shw[wv];
-    const int s = pair / g.Hkv, gh = pair - s * g.Hkv;
+    // (decode: from the grid; a division before the length's load took 0.4 us of 36 a step)
+    const int s = DEC ? (int)blockIdx.z : pair / g.Hkv, gh = DEC ? (int)blockIdx.y : pair - s * g.Hkv;
     // (decode: n_q is the bound on the lengths; one out of range has no tile)
     const int L = DEC ? seq_len[s] : g.pf_pos0 + s + 1;
     const int hn = l & 15, lg = l >> 4;              // MFMA column (head) and k-group of this lane
@@ -2874,7 +2875,7 @@ k_pf_attn(Geo g, qwfn_kv_view v, const float *__restrict__ q, int32_t n_q, const
     const int n = DEC && !(L >= 1 && L <= n_q) ? 0 : min(DEC && !sel ? (L - 1) / g.bt + 1 : nsel[pair], max_sel);
     // this workgroup's part (an even count starts each pair's at another one, see
     // launch_dec_walk) and tiles
-    const int part = !DEC ? 0 : gridDim.x % 2 ? (int)blockIdx.x : (int)((blockIdx.x + blockIdx.y) % gridDim.x);
+    const int part = !DEC ? 0 : gridDim.x % 2 ? (int)blockIdx.x : (int)((blockIdx.x + (uint32_t)pair) % gridDim.x);
     const int t_first = part * split;
     if (DEC && t_first >= n * tpb) return;           // (the whole workgroup) no partial: the merge reads fewer
     const int32_t *selp = sel + (int64_t)pair * max_sel;
@@ -3390,7 +3391,7 @@ hipError_t launch_dec_walk(const Geo &g, const qwfn_kv_view &v, const float *q, 
     const int64_t pairs = (int64_t)g.Hkv * n_seq, cus = device_cus();
     int64_t parts = (ws.n_tiles + tpw - 1) / tpw;
     if (parts % 2 == 0 && (pairs * (parts + 1) + cus - 1) / cus == (pairs * parts + cus - 1) / cus) ++parts;
-    const dim3 grid((unsigned)parts, (unsigned)pairs);
+    const dim3 grid((unsigned)parts, (unsigned)g.Hkv, (unsigned)n_seq);
 #define X(HD_, G_)                                                                                                  \
     if (g.hd == HD_ && g.G == G_) {                                                                                 \
         QWFN_LAUNCH(kTimedAttention, (k_pf_attn<HD_, G_, kPfDecode>), grid, dim3(kPfDecWaves * 64), st, g, v, q,     \

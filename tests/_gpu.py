@@ -161,9 +161,9 @@ def decode_steps(cfg, lengths, steps, seed, dtype=np.float32, zero_pooled=False,
     return outs
 
 
-def graph_grids(fn):
-    """Grid (x, y, z) of each kernel that `fn` (a call on the current stream) captures
-    into a HIP graph."""
+def graph_launches(fn):
+    """(grid (x, y, z), dynamic LDS bytes) of each kernel that `fn` (a call on the current
+    stream) captures into a HIP graph, in order."""
     class Params(ctypes.Structure):
         _fields_ = [("block", ctypes.c_uint * 3), ("extra", ctypes.c_void_p), ("func", ctypes.c_void_p),
                     ("grid", ctypes.c_uint * 3), ("args", ctypes.c_void_p), ("shared", ctypes.c_uint)]
@@ -181,14 +181,14 @@ def graph_grids(fn):
     assert hip.hipGraphGetNodes(raw, None, ctypes.byref(n)) == 0
     nodes = (ctypes.c_void_p * n.value)()
     assert hip.hipGraphGetNodes(raw, nodes, ctypes.byref(n)) == 0
-    grids = []
+    got = []
     for node in nodes:
         p = Params()
         assert hip.hipGraphKernelNodeGetParams(ctypes.c_void_p(node), ctypes.byref(p)) == 0
-        grids.append(tuple(p.grid))
-    return grids
+        got.append((tuple(p.grid), p.shared))
+    return got
 
 
 def graph_nodes(fn):
     """Launches `fn` captures into a HIP graph."""
-    return len(graph_grids(fn))
+    return len(graph_launches(fn))

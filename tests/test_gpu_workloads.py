@@ -31,7 +31,7 @@ import numpy as np
 import pytest
 import torch
 
-from _gpu import assert_close_attn, cfg_of, decode_steps, fill, graph_grids, kv_rows, make_pair, np_of
+from _gpu import assert_close_attn, cfg_of, decode_steps, fill, graph_launches, kv_rows, make_pair, np_of
 from _refs import BASELINE, Cfg
 from qwfnfer_amd import qsa
 
@@ -172,8 +172,8 @@ def test_batched_attention_walks_tiles(cfg, lengths):
 
 
 def _walk_grid(cfg, n_seq, tokens):
-    """Grid of a decode step's attention that walks tiles (parts, (sequence, KV head)), or
-    None where the step launches none."""
+    """Grid of a decode step's attention, the launch before the merge, where it walks tiles:
+    then it asks for no dynamic LDS, as k_dec does.  Else None."""
     c = cfg_of(cfg)
     dev = qsa.KvCache.allocate(c, n_seq, tokens // cfg.page_tokens + 1)
     q = torch.zeros((n_seq, cfg.n_head, cfg.head_dim), device="cuda")
@@ -183,8 +183,9 @@ def _walk_grid(cfg, n_seq, tokens):
     step = lambda: qsa.sparse_attn_decode(dev, q, rows, rows, lens, tokens, ws, out=out)
     step()
     torch.cuda.synchronize()
-    got = [g for g in graph_grids(step) if g[1:] == (n_seq * cfg.n_head_kv, 1)]
-    return got[0] if got else None
+    grid, lds = graph_launches(step)[-2]
+    assert grid[1:] == (cfg.n_head_kv, n_seq)
+    return None if lds else grid
 
 
 @pytest.mark.parametrize("cfg, n_seq, tokens, parts", [
@@ -196,7 +197,7 @@ def test_batched_attention_idle_part_starts_no_round(cfg, n_seq, tokens, parts):
     """Parts a (sequence, KV head): as many as its tiles make, one idle one more where that
     makes the count odd and starts no further round of workgroups on 256 CUs."""
     print(f"parts: {n_seq} sequences of {tokens}, {parts}", flush=True)
-    assert _walk_grid(cfg, n_seq, tokens) == (parts, n_seq * cfg.n_head_kv, 1)
+    assert _walk_grid(cfg, n_seq, tokens) == (parts, cfg.n_head_kv, n_seq)
 
 
 @pytest.mark.parametrize("cfg, n_seq, tokens, walks", [
